@@ -5,21 +5,33 @@
 //
 // Forward: o_i = sum_j p_ij v_j, p_ij = softmax_j(scale * [q_i, 1/scale] . [k_j, bias_j])
 // over the packed rows, the last causal_tail rows causal. With D_i = dO_i . o_i
-// (= sum_j p_ij dO_i . v_j, formed in float32 here) and dS_ij = p_ij (dO_i . v_j - D_i):
+// (= sum_j p_ij dO_i . v_j, formed in float32 here: the rounded forward output would lose the
+// bits that cancel in dS) and dS_ij = p_ij (dO_i . v_j - D_i):
 //   dq_i = scale * sum_j dS_ij k_j      (key features only; the bias coordinate has no gradient)
 //   dk_j = scale * sum_i dS_ij q_i,  dv_j = sum_i p_ij dO_i
 // for the last `grad_rows` packed rows (the in-flight chunk; every row for slot attention).
 //
-// Two launches, both v_mfma_f32_32x32x16_bf16 with the forward's fragment layout:
-//  * dq_kernel: a block owns 128 query rows of one KV group (4 waves x 32, a query per
-//    lane column) and walks the key tiles twice: first the row maximum and sum (the
-//    log-sum-exp) and D, then S^T = K Q^T, dP^T = V dO^T, dS^T and dQ^T += K^T dS^T. It
-//    writes each query's log-sum-exp and D for the second launch.
-//  * dkv_kernel: a block owns 128 gradient rows (a key per lane column) and walks the
-//    query tiles: S = Q K^T, dP = dO V^T, P and dS from the stored statistics, then
-//    dV^T += dO^T P and dK^T += Q^T dS.
-// The P / dS operands are the lanes' own accumulator registers (the k-index permutation of
-// the forward's P^T operand), each as a high and a low bf16 part; accumulation is float32.
+// All products are v_mfma_f32_32x32x16_bf16 with the forward's fragment layout. A wave's own
+// 32 rows (queries for dq, keys for dk / dv) are the B operand and stay in registers for the
+// whole walk; the other side streams through double-buffered LDS tiles of 64 rows, loaded into
+// registers one tile ahead, one barrier per tile. Both operands of a streamed tile come from
+// one row-major copy: as rows by 16-byte reads (S and dP), transposed by ds_read_b64_tr_b16
+// (dQ^T += K^T dS^T, dK^T += Q^T dS, dV^T += dO^T P).
+//  * stats_kernel: the online maximum, sum and sum of p dP of each query over one part of
+//    its key range;
+//  * dq_kernel: the parts combined to the log-sum-exp and D (also stored for dkv_kernel), then
+//    S^T = K Q^T, dP^T = V dO^T, dS^T and dQ^T += K^T dS^T over one part of the key range;
+//  * dkv_kernel: 128 gradient rows per block over one part of the query rows;
+//  * sum_dq_kernel / sum_dkv_kernel: the parts' float32 partials added in part order.
+// The ranges are split so that the launches fill the 256 CUs (bwd_splits). P and dS are the
+// lanes' own accumulator registers (the k-index permutation of the forward's P^T operand), each
+// as a high and a low bf16 part; accumulation is float32.
+//
+// Measured at 2 x 1024 query rows, 16 heads of 128 on 8 groups, 9.3K packed rows and a 1024-row
+// chunk: dq 264 us and statistics 185 us (one 128-row block of four waves, tiles staged by element
+// and re-read from LDS as both operands: 1880 us together), dk / dv 99 us with its rows loaded as
+// 16-byte units (1224 us by element); bound by matrix-core issue and the exponentials of the two
+// waves of a SIMD running in step.
 #include <algorithm>
 
 #include "route.hpp"
@@ -32,25 +44,33 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 128;       // query rows (dq) / gradient rows (dkv) per block
-constexpr int kTile = 64;        // key rows (dq) / query rows (dkv) per staged tile
-constexpr int kMaxSteps = 9;     // 16-wide steps of the packed width (<= 144)
-constexpr int kLdK = 152;        // row stride of row-major Q / K tiles (bf16)
-constexpr int kLdD = 136;        // row stride of row-major dO / V tiles (dv <= 128)
-constexpr int kLdT = kTile + 8;  // row stride of transposed tiles
-constexpr int kMaxBlk = 4;       // 32-row blocks of dk / dv (<= 128)
+constexpr int kQWaves = 8;                // waves per query block (two per SIMD), 32 queries each
+constexpr int kQRows = 32 * kQWaves;
+constexpr int kKWaves = 4;                // waves per gradient-row block: dk and dv accumulators take one wave per SIMD
+constexpr int kKRows = 32 * kKWaves;
+constexpr int kTile = 64;                 // streamed rows per tile
+constexpr int kLdK = 152;                 // row stride of packed-key / query tiles (bf16; 16-byte reads of 8 rows: 8 bank groups)
+constexpr int kLdD = 136;                 // row stride of value / dO tiles (dv <= 128)
+constexpr int kMaxSplits = 16;
 constexpr float kLog2e = 1.44269504088896341f;
 
 __device__ __forceinline__ bf16x8 load8(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
-// A operand of a transposed tile (rows x tile columns), columns in the
-// permuted order 16 st + 8 (j / 4) + 4 h + j % 4 of step st.
-__device__ __forceinline__ bf16x8 load_t(const uint16_t* base, int row, int st, int h) {
-  const uint16_t* r = base + row * kLdT + 16 * st + 4 * h;
-  const uint2 x0 = *reinterpret_cast<const uint2*>(r);
-  const uint2 x1 = *reinterpret_cast<const uint2*>(r + 8);
-  return __builtin_bit_cast(bf16x8, make_uint4(x0.x, x0.y, x1.x, x1.y));
+// Transposed A operand of a row-major tile: for feature f0 + lane % 32, rows 16 st + 8 (j / 4) +
+// 4 (lane / 32) + j % 4 (the order of the accumulator registers' elements). ds_read_b64_tr_b16
+// turns a 16-lane group's 4 rows x 16 features (lane i reads row i / 4, features 4 (i % 4) .. + 4)
+// into 4 rows of feature i per lane.
+template <int LD>
+__device__ __forceinline__ bf16x8 load_tr(const uint16_t* tile, int f0, int st) {
+  typedef __attribute__((address_space(3))) s16x4* lds4;
+  const int l = lane_id(), i = l & 15, h = l >> 5;
+  const uint16_t* p = tile + (16 * st + 4 * h + (i >> 2)) * LD + f0 + (l & 16) + 4 * (i & 3);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p + 8 * LD));
+  const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  return __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, y.x, y.y));
 }
 
 // B operand of step st from accumulator blocks acc[2] (elements 8 (st % 2) .. + 8 of block
@@ -74,119 +94,189 @@ __device__ __forceinline__ int packed_total(const logkv_attention_args& a, const
   return min(*width_ptr + a.tail + (a.alpha_count_dev ? *a.alpha_count_dev : 0), a.cap);
 }
 
+// Features d .. d + 7 of a strided bf16 row (those past n zero): one 16-byte load where the rows
+// are 16-byte aligned (`vec`; n is a multiple of 8), else by element.
+__device__ __forceinline__ uint4 row_unit(const LOGKV_G uint16_t* row, int d, int n, bool vec) {
+  if (d >= n) return make_uint4(0, 0, 0, 0);
+  if (vec) return *(const LOGKV_G uint4*)(row + d);
+  uint32_t x[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = row[d + 2 * j] | (static_cast<uint32_t>(row[d + 2 * j + 1]) << 16);
+  return make_uint4(x[0], x[1], x[2], x[3]);
+}
+
+// The query row [q, 1/scale, 0...], features d .. d + 7 (dk is a multiple of 8).
+__device__ __forceinline__ uint4 query_unit(const logkv_attention_args& a, const LOGKV_G uint16_t* row, int d, bool vec) {
+  if (d == a.dk) return make_uint4(f32_to_bf16(a.inv_scale_bf16), 0, 0, 0);
+  return row_unit(row, d, a.dk, vec);
+}
+
+// Workgroups go to the 8 XCDs round robin: dispatched block n takes logical block (n % 8) (N / 8)
+// + n / 8 (N a multiple of 8), so the blocks of a lane, which stream the same rows, share one L2.
+struct BwdBlock {
+  int x, split, lane;
+};
+__device__ __forceinline__ BwdBlock bwd_block() {
+  const int nx = static_cast<int>(gridDim.x), ny = static_cast<int>(gridDim.y);
+  const int n = nx * ny * static_cast<int>(gridDim.z);
+  int lin = static_cast<int>(blockIdx.x) + nx * (static_cast<int>(blockIdx.y) + ny * static_cast<int>(blockIdx.z));
+  if (n % 8 == 0) lin = (lin % 8) * (n / 8) + lin / 8;
+  return BwdBlock{lin % nx, (lin / nx) % ny, lin / (nx * ny)};
+}
+
+struct BwdLayout {
+  int q_splits;    // parts of the key range (stats_kernel, dq_kernel)
+  int k_splits;    // parts of the query rows (dkv_kernel)
+  int vec_q, vec_do, vec_dq;   // rows of q / dO 16-byte aligned, of dq 8-byte aligned
+  float* stats;    // [lanes, nq, 2]: log-sum-exp, D
+  float* part;     // [lanes, q_splits, nq, 4]: maximum, sum, sum of p dP
+  float* grad;     // partials of dq [lanes, q_splits, nq, dk], then of dk / dv [lanes, k_splits, grad_rows, dk + dv]
+};
+
+// A block's streamed K / V tiles: rows t0 .. of the lane's packed rows, those past `stop` zero.
+template <int NKS, int NDV, int THREADS>
+struct KvTiles {
+  static constexpr int kUnitsK = 2 * NKS, kUnitsV = 4 * NDV;
+  static constexpr int kTasksK = (kTile * kUnitsK + THREADS - 1) / THREADS, kTasksV = (kTile * kUnitsV + THREADS - 1) / THREADS;
+  uint4 kx[kTasksK], vx[kTasksV];
+  __device__ __forceinline__ void load(const logkv_attention_args& a, const LOGKV_G uint16_t* kbase,
+                                       const LOGKV_G uint16_t* vbase, int t0, int stop) {
+#pragma unroll
+    for (int q = 0; q < kTasksK; ++q) {
+      const int i = threadIdx.x + THREADS * q, r = i / kUnitsK, u = i % kUnitsK;
+      const bool on = r < kTile && t0 + r < stop && 8 * u < a.dim;
+      kx[q] = *(const LOGKV_G uint4*)(kbase + static_cast<int64_t>(on ? t0 + r : t0) * a.dim + (on ? 8 * u : 0));
+      if (!on) kx[q] = make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < kTasksV; ++q) {
+      const int i = threadIdx.x + THREADS * q, r = i / kUnitsV, u = i % kUnitsV;
+      const bool on = r < kTile && t0 + r < stop && 8 * u < a.dv;
+      vx[q] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(on ? t0 + r : t0) * a.dim + (on ? 8 * u : 0));
+      if (!on) vx[q] = make_uint4(0, 0, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void store(uint16_t* k_s, uint16_t* v_s) const {
+#pragma unroll
+    for (int q = 0; q < kTasksK; ++q) {
+      const int i = threadIdx.x + THREADS * q, r = i / kUnitsK, u = i % kUnitsK;
+      if (r < kTile) *reinterpret_cast<uint4*>(k_s + r * kLdK + 8 * u) = kx[q];
+    }
+#pragma unroll
+    for (int q = 0; q < kTasksV; ++q) {
+      const int i = threadIdx.x + THREADS * q, r = i / kUnitsV, u = i % kUnitsV;
+      if (r < kTile) *reinterpret_cast<uint4*>(v_s + r * kLdD + 8 * u) = vx[q];
+    }
+  }
+};
+
+// One query block over one part of its key range: the own query and dO fragments, and a walk of
+// the key tiles that hands f(s, dp, t0, k tile) the tile's masked scores S^T and dP^T.
+template <int NKS, int NDV>
+struct QueryWalk {
+  int lane_ix, b, qi, head, t, total, tail0, k_begin, k_stop;
+  bool q_ok;
+  bf16x8 qf[NKS], df[2 * NDV];
+
+  __device__ __forceinline__ QueryWalk(const logkv_attention_args& a, const int32_t* width_ptr,
+                                       const logkv_attention_grad_args& gr, const BwdLayout& lay, const BwdBlock& id) {
+    const int G = a.n_groups, rep = a.n_heads / G, nq = rep * a.tq;
+    lane_ix = id.lane;
+    b = lane_ix / G;
+    const int w = wave_id(), l = lane_id(), h = l >> 5, col = l & 31;
+    qi = id.x * kQRows + w * 32 + col;
+    q_ok = qi < nq;
+    const int qc = q_ok ? qi : nq - 1;
+    head = (lane_ix % G) * rep + qc / a.tq;
+    t = qc % a.tq;
+    total = packed_total(a, width_ptr);
+    tail0 = total - a.causal_tail;
+    // Last key row any query of the block can see, and this block's part of the range in whole tiles.
+    const int q_first = id.x * kQRows, q_last = min(q_first + kQRows, nq) - 1;
+    const int t_max = q_first / a.tq == q_last / a.tq ? q_last % a.tq : a.tq - 1;
+    const int key_end = a.causal_tail ? min(total, tail0 + t_max + 1) : total;
+    const int tiles = (key_end + kTile - 1) / kTile, per = (tiles + lay.q_splits - 1) / lay.q_splits;
+    k_begin = min(id.split * per, tiles) * kTile;
+    k_stop = min(min((id.split + 1) * per, tiles) * kTile, key_end);
+    const LOGKV_G uint16_t* qrow = gp(a.q) + b * a.q_sb + head * a.q_sh + t * a.q_st;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+      qf[ks] = __builtin_bit_cast(bf16x8, query_unit(a, qrow, 16 * ks + 8 * h, lay.vec_q));
+    const LOGKV_G uint16_t* drow = gp(gr.dout) + b * gr.do_sb + head * gr.do_sh + t * gr.do_st;
+#pragma unroll
+    for (int st = 0; st < 2 * NDV; ++st)
+      df[st] = __builtin_bit_cast(bf16x8, row_unit(drow, 16 * st + 8 * h, a.dv, lay.vec_do));
+  }
+
+  template <class F>
+  __device__ __forceinline__ void walk(const logkv_attention_args& a, uint16_t (*k_s)[kTile * kLdK],
+                                       uint16_t (*v_s)[kTile * kLdD], F&& f) const {
+    const LOGKV_G uint16_t* kbase = gp(a.k) + static_cast<int64_t>(lane_ix) * a.cap * a.dim;
+    const LOGKV_G uint16_t* vbase = gp(a.v) + static_cast<int64_t>(lane_ix) * a.cap * a.dim;
+    const int l = lane_id(), h = l >> 5, col = l & 31;
+    const int n = k_begin < k_stop ? (k_stop - k_begin + kTile - 1) / kTile : 0;
+    KvTiles<NKS, NDV, 64 * kQWaves> tiles;
+    if (n > 0) {
+      tiles.load(a, kbase, vbase, k_begin, k_stop);
+      tiles.store(k_s[0], v_s[0]);
+      if (n > 1) tiles.load(a, kbase, vbase, k_begin + kTile, k_stop);
+    }
+    __syncthreads();
+    for (int it = 0; it < n; ++it) {
+      const int t0 = k_begin + it * kTile, bf = it & 1;
+      const uint16_t* kt = k_s[bf];
+      const uint16_t* vt = v_s[bf];
+      f32x16 s[2], dp[2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[kb][i] = 0.f;
+          dp[kb][i] = 0.f;
+        }
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(kt + (32 * kb + col) * kLdK + 16 * ks + 8 * h), qf[ks],
+                                                          s[kb], 0, 0, 0);
+#pragma unroll
+      for (int st = 0; st < 2 * NDV; ++st)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          dp[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(vt + (32 * kb + col) * kLdD + 16 * st + 8 * h), df[st],
+                                                           dp[kb], 0, 0, 0);
+      // Tiles with rows past the end or past some query's causal limit (uniform over the block).
+      if (t0 + kTile > k_stop || (a.causal_tail && t0 + kTile > tail0)) {
+        const int lim = (a.causal_tail ? min(k_stop, tail0 + t + 1) : k_stop) - t0 - 4 * h;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[kb][i] = 32 * kb + 8 * (i / 4) + (i % 4) < lim ? s[kb][i] : -__builtin_inff();
+      }
+      f(s, dp, kt);
+      if (it + 1 < n) {
+        tiles.store(k_s[bf ^ 1], v_s[bf ^ 1]);
+        if (it + 2 < n) tiles.load(a, kbase, vbase, t0 + 2 * kTile, k_stop);
+      }
+      __syncthreads();
+    }
+  }
+};
+
 }  // namespace
 
-__global__ __launch_bounds__(256, 1) void dq_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
-                                                    logkv_attention_grad_args gr, float* __restrict__ stats) {
-  __shared__ __align__(16) uint16_t q_s[kRows * kLdK];
-  __shared__ __align__(16) uint16_t do_s[kRows * kLdD];
-  __shared__ __align__(16) uint16_t k_s[kTile * kLdK];
-  __shared__ __align__(16) uint16_t kt_s[kMaxBlk * 32 * kLdT];
-  __shared__ __align__(16) uint16_t v_s[kTile * kLdD];
-  const int lane_ix = blockIdx.y, G = a.n_groups;
-  const int b = lane_ix / G, g = lane_ix % G;
-  const int rep = a.n_heads / G, nq = rep * a.tq;
-  const int w = wave_id(), l = lane_id(), h = l >> 5, col = l & 31;
-  const int dim = a.dim, nks = (dim + 15) / 16, nvs = a.dv / 16, ndk = (a.dk + 31) / 32;
-  const int qi = blockIdx.x * kRows + w * 32 + col;
-  const bool q_ok = qi < nq;
-  const int qc = q_ok ? qi : nq - 1;
-  const int head = g * rep + qc / a.tq, t = qc % a.tq;
-  const int total = packed_total(a, width_ptr);
-  const int tail0 = total - a.causal_tail;
-  const int q_first = blockIdx.x * kRows, q_last = min(q_first + kRows, nq) - 1;
-  const int t_max = q_first / a.tq == q_last / a.tq ? q_last % a.tq : a.tq - 1;
-  const int key_end = a.causal_tail ? min(total, tail0 + t_max + 1) : total;
+template <int NKS, int NDV>
+__global__ __launch_bounds__(64 * kQWaves, 2) void stats_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
+                                                       logkv_attention_grad_args gr, BwdLayout lay) {
+  __shared__ __align__(16) uint16_t k_s[2][kTile * kLdK];
+  __shared__ __align__(16) uint16_t v_s[2][kTile * kLdD];
+  const BwdBlock id = bwd_block();
+  const QueryWalk<NKS, NDV> me(a, width_ptr, gr, lay, id);
   const float c2 = a.scale * kLog2e;
-
-  for (int i = threadIdx.x; i < kRows * kLdK; i += blockDim.x) {
-    const int r = i / kLdK, d = i - r * kLdK;
-    const int qr = min(q_first + r, nq - 1);
-    const int hr = g * rep + qr / a.tq, tr = qr % a.tq;
-    const float x = d < a.dk ? bf16_to_f32(gp(a.q)[b * a.q_sb + hr * a.q_sh + tr * a.q_st + (d < a.dk ? d : 0)])
-                             : (d == a.dk ? a.inv_scale_bf16 : 0.f);
-    q_s[i] = f32_to_bf16(x);
-  }
-  for (int i = threadIdx.x; i < kRows * kLdD; i += blockDim.x) {
-    const int r = i / kLdD, d = i - r * kLdD;
-    const int qr = min(q_first + r, nq - 1);
-    const int hr = g * rep + qr / a.tq, tr = qr % a.tq;
-    do_s[i] = d < a.dv ? gp(gr.dout)[b * gr.do_sb + hr * gr.do_sh + tr * gr.do_st + (d < a.dv ? d : 0)] : 0;
-  }
-  for (int i = threadIdx.x; i < kTile * (kLdK - dim); i += blockDim.x) {
-    const int r = i / (kLdK - dim), c = dim + i % (kLdK - dim);
-    k_s[r * kLdK + c] = 0;
-  }
-  const LOGKV_G uint16_t* kbase = gp(a.k) + static_cast<int64_t>(lane_ix) * a.cap * dim;
-  const LOGKV_G uint16_t* vbase = gp(a.v) + static_cast<int64_t>(lane_ix) * a.cap * dim;
-  const int units = dim / 8, vunits = a.dv / 8;
-
-  auto scores = [&](f32x16 (&s)[2]) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[kb][i] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < kMaxSteps; ++ks)
-        if (ks < nks)
-          s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(k_s + (32 * kb + col) * kLdK + 16 * ks + 8 * h),
-                                                          load8(q_s + (32 * w + col) * kLdK + 16 * ks + 8 * h),
-                                                          s[kb], 0, 0, 0);
-    }
-  };
-  auto mask = [&](f32x16 (&s)[2], int t0, int rows) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = t0 + 32 * kb + 8 * (i / 4) + 4 * h + (i % 4);
-        const bool masked = key >= t0 + rows || (a.causal_tail && key >= tail0 && key - tail0 > t);
-        s[kb][i] = masked ? -__builtin_inff() : s[kb][i];
-      }
-  };
-  auto stage_k = [&](int t0, int rows) {
-    for (int i = threadIdx.x; i < kTile * units; i += blockDim.x) {
-      const int r = i / units, u = i - r * units;
-      uint4 x = make_uint4(0, 0, 0, 0);
-      if (r < rows) x = *(const LOGKV_G uint4*)(kbase + static_cast<int64_t>(t0 + r) * dim + 8 * u);
-      *reinterpret_cast<uint4*>(k_s + r * kLdK + 8 * u) = x;
-    }
-  };
-  auto stage_v = [&](int t0, int rows) {
-    for (int i = threadIdx.x; i < kTile * vunits; i += blockDim.x) {
-      const int r = i / vunits, u = i - r * vunits;
-      uint4 x = make_uint4(0, 0, 0, 0);
-      if (r < rows) x = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + r) * dim + 8 * u);
-      *reinterpret_cast<uint4*>(v_s + r * kLdD + 8 * u) = x;
-    }
-  };
-  // dP^T = V dO^T for the staged tile (keys x this lane's query).
-  auto dscores = [&](f32x16 (&dp)[2]) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dp[kb][i] = 0.f;
-      for (int st = 0; st < nvs; ++st)
-        dp[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(v_s + (32 * kb + col) * kLdD + 16 * st + 8 * h),
-                                                         load8(do_s + (32 * w + col) * kLdD + 16 * st + 8 * h),
-                                                         dp[kb], 0, 0, 0);
-    }
-  };
-
-  // Pass 1: the log-sum-exp of this lane's query (base 2, scaled by c2) and
-  // D = dO . o = sum_j p_j dP_j, accumulated with the same online rescaling in
-  // float32 (the rounded forward output would lose the bits that cancel in dS).
   float m = -__builtin_inff(), lsum = 0.f, dacc = 0.f;
-  for (int t0 = 0; t0 < key_end; t0 += kTile) {
-    const int rows = min(kTile, key_end - t0);
-    __syncthreads();
-    stage_k(t0, rows);
-    stage_v(t0, rows);
-    __syncthreads();
-    f32x16 s[2], dp[2];
-    scores(s);
-    dscores(dp);
-    mask(s, t0, rows);
+  me.walk(a, k_s, v_s, [&](f32x16 (&s)[2], f32x16 (&dp)[2], const uint16_t*) {
     float mx = -__builtin_inff();
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -195,53 +285,59 @@ __global__ __launch_bounds__(256, 1) void dq_kernel(logkv_attention_args a, cons
     mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
     const float m_new = fmaxf(m, mx * c2);
     const float mb = m_new == -__builtin_inff() ? 0.f : m_new;
-    float sum = 0.f, dsum_t = 0.f;
+    float sum = 0.f, dsum = 0.f;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][i], c2, -mb));
         sum += p;
-        dsum_t += p * dp[kb][i];
+        dsum = __builtin_fmaf(p, dp[kb][i], dsum);
       }
-    sum += __shfl_xor(sum, 32, kWave);
-    dsum_t += __shfl_xor(dsum_t, 32, kWave);
     const float corr = __builtin_amdgcn_exp2f(m - mb);
-    lsum = lsum * corr + sum;
-    dacc = dacc * corr + dsum_t;
+    lsum = lsum * corr + sum;     // this lane's half of the keys; the halves are added below
+    dacc = dacc * corr + dsum;
     m = m_new;
+  });
+  lsum += __shfl_xor(lsum, 32, kWave);
+  dacc += __shfl_xor(dacc, 32, kWave);
+  if (me.q_ok && lane_id() < 32) {
+    const int nq = a.n_heads / a.n_groups * a.tq;
+    *reinterpret_cast<float4*>(lay.part + ((static_cast<int64_t>(id.lane) * lay.q_splits + id.split) * nq + me.qi) * 4) =
+        make_float4(m, lsum, dacc, 0.f);
+  }
+}
+
+template <int NKS, int NDV>
+__global__ __launch_bounds__(64 * kQWaves, 2) void dq_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
+                                                    logkv_attention_grad_args gr, BwdLayout lay) {
+  __shared__ __align__(16) uint16_t k_s[2][kTile * kLdK];
+  __shared__ __align__(16) uint16_t v_s[2][kTile * kLdD];
+  const BwdBlock id = bwd_block();
+  const QueryWalk<NKS, NDV> me(a, width_ptr, gr, lay, id);
+  const int nq = a.n_heads / a.n_groups * a.tq, h = lane_id() >> 5;
+  const float c2 = a.scale * kLog2e;
+  // The parts of this lane's query, combined in part order.
+  const float4* pp = reinterpret_cast<const float4*>(lay.part) +
+                     static_cast<int64_t>(id.lane) * lay.q_splits * nq + (me.q_ok ? me.qi : nq - 1);
+  float m = -__builtin_inff(), lsum = 0.f, dacc = 0.f;
+  for (int sp = 0; sp < lay.q_splits; ++sp) m = fmaxf(m, pp[static_cast<int64_t>(sp) * nq].x);
+  for (int sp = 0; sp < lay.q_splits; ++sp) {
+    const float4 x = pp[static_cast<int64_t>(sp) * nq];
+    const float f = x.x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(x.x - m);
+    lsum += x.y * f;
+    dacc += x.z * f;
   }
   const float lse = lsum > 0.f ? m + __log2f(lsum) : 0.f;
   const float dsum = lsum > 0.f ? dacc / lsum : 0.f;
-  if (q_ok && h == 0) {
-    stats[(static_cast<int64_t>(lane_ix) * nq + qi) * 2] = lse;
-    stats[(static_cast<int64_t>(lane_ix) * nq + qi) * 2 + 1] = dsum;
-  }
-
-  // Pass 2: dQ^T += K^T dS^T.
-  f32x16 dq[kMaxBlk];
+  if (id.split == 0 && me.q_ok && h == 0)
+    *reinterpret_cast<float2*>(lay.stats + (static_cast<int64_t>(id.lane) * nq + me.qi) * 2) = make_float2(lse, dsum);
+  f32x16 dq[NDV];
 #pragma unroll
-  for (int blk = 0; blk < kMaxBlk; ++blk)
+  for (int blk = 0; blk < NDV; ++blk)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dq[blk][i] = 0.f;
-  for (int t0 = 0; t0 < key_end; t0 += kTile) {
-    const int rows = min(kTile, key_end - t0);
-    __syncthreads();
-    stage_k(t0, rows);
-    // K^T (key features only) and V, row-major.
-    for (int i = threadIdx.x; i < kTile * (a.dk / 2); i += blockDim.x) {
-      const int r = i % kTile, d2 = i / kTile;
-      uint32_t x = 0;
-      if (r < rows) x = *(const LOGKV_G uint32_t*)(kbase + static_cast<int64_t>(t0 + r) * dim + 2 * d2);
-      kt_s[(2 * d2) * kLdT + r] = static_cast<uint16_t>(x);
-      kt_s[(2 * d2 + 1) * kLdT + r] = static_cast<uint16_t>(x >> 16);
-    }
-    stage_v(t0, rows);
-    __syncthreads();
-    f32x16 s[2], dp[2];
-    scores(s);
-    mask(s, t0, rows);
-    dscores(dp);
+  me.walk(a, k_s, v_s, [&](f32x16 (&s)[2], f32x16 (&dp)[2], const uint16_t* kt) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -253,145 +349,214 @@ __global__ __launch_bounds__(256, 1) void dq_kernel(logkv_attention_args a, cons
     for (int st = 0; st < 4; ++st) {
       bf16x8 dh, dl;
       regs_b(dp, st, dh, dl);
+      bf16x8 kf[NDV];
 #pragma unroll
-      for (int blk = 0; blk < kMaxBlk; ++blk)
-        if (blk < ndk) {
-          const bf16x8 kf = load_t(kt_s, 32 * blk + col, st, h);
-          dq[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, dh, dq[blk], 0, 0, 0);
-          dq[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, dl, dq[blk], 0, 0, 0);
-        }
+      for (int blk = 0; blk < NDV; ++blk) kf[blk] = load_tr<kLdK>(kt, 32 * blk, st);
+#pragma unroll
+      for (int blk = 0; blk < NDV; ++blk) dq[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[blk], dh, dq[blk], 0, 0, 0);
+#pragma unroll
+      for (int blk = 0; blk < NDV; ++blk) dq[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[blk], dl, dq[blk], 0, 0, 0);
     }
-  }
-  if (!q_ok) return;
-  LOGKV_G uint16_t* drow = gp(gr.dq) + b * gr.dq_sb + head * gr.dq_sh + t * gr.dq_st;
+  });
+  if (!me.q_ok) return;
+  if (lay.q_splits > 1) {
+    float* out = lay.grad + ((static_cast<int64_t>(id.lane) * lay.q_splits + id.split) * nq + me.qi) * a.dk;
 #pragma unroll
-  for (int blk = 0; blk < kMaxBlk; ++blk)
-    if (blk < ndk)
+    for (int blk = 0; blk < NDV; ++blk)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int d = 32 * blk + 8 * (i / 4) + 4 * h + (i % 4);
-        if (d < a.dk) drow[d] = f32_to_bf16(dq[blk][i] * a.scale);
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int d = 32 * blk + 8 * i4 + 4 * h;
+        if (d < a.dk)
+          *reinterpret_cast<float4*>(out + d) =
+              make_float4(dq[blk][4 * i4], dq[blk][4 * i4 + 1], dq[blk][4 * i4 + 2], dq[blk][4 * i4 + 3]);
       }
+    return;
+  }
+  LOGKV_G uint16_t* drow = gp(gr.dq) + me.b * gr.dq_sb + me.head * gr.dq_sh + me.t * gr.dq_st;
+#pragma unroll
+  for (int blk = 0; blk < NDV; ++blk)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int d = 32 * blk + 8 * (i / 4) + 4 * h + (i % 4);
+      if (d < a.dk) drow[d] = f32_to_bf16(dq[blk][i] * a.scale);
+    }
 }
 
-__global__ __launch_bounds__(256, 1) void dkv_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
-                                                     logkv_attention_grad_args gr, const float* __restrict__ stats) {
-  __shared__ __align__(16) uint16_t ks_s[kRows * kLdK];
-  __shared__ __align__(16) uint16_t vs_s[kRows * kLdD];
-  __shared__ __align__(16) uint16_t q_t[kTile * kLdK];
-  __shared__ __align__(16) uint16_t qt_t[kMaxBlk * 32 * kLdT];
-  __shared__ __align__(16) uint16_t do_t[kTile * kLdD];
-  __shared__ __align__(16) uint16_t dot_t[kMaxBlk * 32 * kLdT];
-  __shared__ float st_s[kTile][2];
-  const int lane_ix = blockIdx.y, G = a.n_groups;
-  const int b = lane_ix / G, g = lane_ix % G;
+// dq = scale * (the parts' partials in part order): one thread per query and four features.
+__global__ __launch_bounds__(256) void sum_dq_kernel(logkv_attention_args a, logkv_attention_grad_args gr, BwdLayout lay) {
+  const int nq = a.n_heads / a.n_groups * a.tq, units = a.dk / 4;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nq * units) return;
+  const int qi = i / units, d = 4 * (i % units), lane_ix = blockIdx.y;
+  const float* part = lay.grad + (static_cast<int64_t>(lane_ix) * lay.q_splits * nq + qi) * a.dk + d;
+  float x[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int sp = 0; sp < lay.q_splits; ++sp) {
+    const float4 p = *reinterpret_cast<const float4*>(part + static_cast<int64_t>(sp) * nq * a.dk);
+    x[0] += p.x;
+    x[1] += p.y;
+    x[2] += p.z;
+    x[3] += p.w;
+  }
+  uint32_t o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(x[j] * a.scale);
+  const int b = lane_ix / a.n_groups, head = (lane_ix % a.n_groups) * (a.n_heads / a.n_groups) + qi / a.tq, t = qi % a.tq;
+  LOGKV_G uint16_t* row = gp(gr.dq) + b * gr.dq_sb + head * gr.dq_sh + t * gr.dq_st + d;
+  if (lay.vec_dq) {
+    *(LOGKV_G uint2*)(row) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) row[j] = static_cast<uint16_t>(o[j]);
+  }
+}
+
+template <int NKS, int NDV>
+__global__ __launch_bounds__(64 * kKWaves, 1) void dkv_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
+                                                     logkv_attention_grad_args gr, BwdLayout lay) {
+  constexpr int kThreads = 64 * kKWaves, kUnitsQ = 2 * NKS, kUnitsD = 4 * NDV;
+  constexpr int kTasksQ = (kTile * kUnitsQ + kThreads - 1) / kThreads, kTasksD = (kTile * kUnitsD + kThreads - 1) / kThreads;
+  __shared__ __align__(16) uint16_t q_s[2][kTile * kLdK];
+  __shared__ __align__(16) uint16_t d_s[2][kTile * kLdD];
+  __shared__ __align__(16) float lse_s[2][kTile];
+  __shared__ __align__(16) float dsum_s[2][kTile];
+  __shared__ __align__(16) int t_s[2][kTile];
+  const BwdBlock id = bwd_block();
+  const int lane_ix = id.lane, G = a.n_groups, b = lane_ix / G, g = lane_ix % G;
   const int rep = a.n_heads / G, nq = rep * a.tq;
-  const int w = wave_id(), l = lane_id(), h = l >> 5, col = l & 31;
-  const int dim = a.dim, nks = (dim + 15) / 16, ndv = a.dv / 32, nvs = a.dv / 16, ndk = (a.dk + 31) / 32;
+  const int w = wave_id(), l = lane_id(), h = l >> 5, col = l & 31, tid = static_cast<int>(threadIdx.x);
   const int total = packed_total(a, width_ptr);
   const int tail0 = total - a.causal_tail;
   const int first = total - gr.grad_rows;                // first gradient row
-  const int r_first = first + blockIdx.x * kRows;
+  const int r_first = first + id.x * kKRows;
   const int key = r_first + w * 32 + col;                  // this lane's key row
-  const bool key_ok = key < total && key >= 0;
+  const bool key_ok = key < total && key >= 0 && key >= first;
   const float c2 = a.scale * kLog2e;
-  const LOGKV_G uint16_t* kbase = gp(a.k) + static_cast<int64_t>(lane_ix) * a.cap * dim;
-  const LOGKV_G uint16_t* vbase = gp(a.v) + static_cast<int64_t>(lane_ix) * a.cap * dim;
-  const int units = dim / 8, vunits = a.dv / 8;
-  for (int i = threadIdx.x; i < kRows * units; i += blockDim.x) {
-    const int r = i / units, u = i - r * units;
-    const int kr = r_first + r;
-    uint4 x = make_uint4(0, 0, 0, 0);
-    if (kr < total && kr >= 0) x = *(const LOGKV_G uint4*)(kbase + static_cast<int64_t>(kr) * dim + 8 * u);
-    *reinterpret_cast<uint4*>(ks_s + r * kLdK + 8 * u) = x;
-  }
-  for (int i = threadIdx.x; i < kRows * (kLdK - dim); i += blockDim.x) {
-    const int r = i / (kLdK - dim), c = dim + i % (kLdK - dim);
-    ks_s[r * kLdK + c] = 0;
-  }
-  for (int i = threadIdx.x; i < kRows * vunits; i += blockDim.x) {
-    const int r = i / vunits, u = i - r * vunits;
-    const int kr = r_first + r;
-    uint4 x = make_uint4(0, 0, 0, 0);
-    if (kr < total && kr >= 0) x = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(kr) * dim + 8 * u);
-    *reinterpret_cast<uint4*>(vs_s + r * kLdD + 8 * u) = x;
-  }
-  for (int i = threadIdx.x; i < kTile * (kLdK - dim); i += blockDim.x) {
-    const int r = i / (kLdK - dim), c = dim + i % (kLdK - dim);
-    q_t[r * kLdK + c] = 0;
-  }
-  // The smallest causal index of this block's rows: query tiles whose every t is
-  // below it see none of them.
-  const int block_min_t = a.causal_tail ? max(0, r_first - tail0) : 0;
-  f32x16 dk[kMaxBlk], dv[kMaxBlk];
+  // The lane's own key and value as B fragments (columns past the packed width / dv zero).
+  bf16x8 kf[NKS], vf[2 * NDV];
+  {
+    const int64_t row = (static_cast<int64_t>(lane_ix) * a.cap + (key_ok ? key : 0)) * a.dim;
 #pragma unroll
-  for (int blk = 0; blk < kMaxBlk; ++blk)
+    for (int ks = 0; ks < NKS; ++ks)
+      kf[ks] = __builtin_bit_cast(bf16x8, row_unit(gp(a.k) + row, 16 * ks + 8 * h, a.dim, true));
+#pragma unroll
+    for (int st = 0; st < 2 * NDV; ++st)
+      vf[st] = __builtin_bit_cast(bf16x8, row_unit(gp(a.v) + row, 16 * st + 8 * h, a.dv, true));
+  }
+  // Query tiles of this part whose last causal index reaches the block's first row: a tile
+  // all of whose queries come before every row of the block has no visible pair.
+  const int tiles = (nq + kTile - 1) / kTile, per = (tiles + lay.k_splits - 1) / lay.k_splits;
+  const int tile_end = min((id.split + 1) * per, tiles);
+  const int min_t = a.causal_tail ? r_first - tail0 : 0;
+  auto next_tile = [&](int tile) {
+    for (; tile < tile_end; ++tile) {
+      const int q0 = tile * kTile, qe = min(q0 + kTile, nq) - 1;
+      if (!a.causal_tail || (q0 / a.tq == qe / a.tq ? qe % a.tq : a.tq - 1) >= min_t) break;
+    }
+    return tile;
+  };
+  uint4 qx[kTasksQ], dx[kTasksD];
+  float lse_x = 0.f, dsum_x = 0.f;
+  int t_x = 0;
+  auto load = [&](int tile) {
+    const int q0 = tile * kTile;
+    auto row_of = [&](int r, int64_t sb, int64_t sh, int64_t st) {
+      const int qr = min(q0 + r, nq - 1);
+      return b * sb + (g * rep + qr / a.tq) * sh + (qr % a.tq) * st;
+    };
+#pragma unroll
+    for (int q = 0; q < kTasksQ; ++q) {
+      const int i = tid + kThreads * q, r = min(i / kUnitsQ, kTile - 1), u = i % kUnitsQ;
+      qx[q] = query_unit(a, gp(a.q) + row_of(r, a.q_sb, a.q_sh, a.q_st), 8 * u, lay.vec_q);
+      if (q0 + r >= nq) qx[q] = make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < kTasksD; ++q) {
+      const int i = tid + kThreads * q, r = min(i / kUnitsD, kTile - 1), u = i % kUnitsD;
+      dx[q] = row_unit(gp(gr.dout) + row_of(r, gr.do_sb, gr.do_sh, gr.do_st), 8 * u, a.dv, lay.vec_do);
+      if (q0 + r >= nq) dx[q] = make_uint4(0, 0, 0, 0);
+    }
+    if (tid < kTile) {
+      const int qr = min(q0 + tid, nq - 1);
+      const float2 x = *reinterpret_cast<const float2*>(lay.stats + (static_cast<int64_t>(lane_ix) * nq + qr) * 2);
+      lse_x = q0 + tid < nq ? x.x : __builtin_inff();   // rows past the queries: p = 2^(-inf) = 0
+      dsum_x = x.y;
+      t_x = qr % a.tq;
+    }
+  };
+  auto store = [&](int bf) {
+#pragma unroll
+    for (int q = 0; q < kTasksQ; ++q) {
+      const int i = tid + kThreads * q, r = i / kUnitsQ, u = i % kUnitsQ;
+      if (r < kTile) *reinterpret_cast<uint4*>(&q_s[bf][r * kLdK + 8 * u]) = qx[q];
+    }
+#pragma unroll
+    for (int q = 0; q < kTasksD; ++q) {
+      const int i = tid + kThreads * q, r = i / kUnitsD, u = i % kUnitsD;
+      if (r < kTile) *reinterpret_cast<uint4*>(&d_s[bf][r * kLdD + 8 * u]) = dx[q];
+    }
+    if (tid < kTile) {
+      lse_s[bf][tid] = lse_x;
+      dsum_s[bf][tid] = dsum_x;
+      t_s[bf][tid] = t_x;
+    }
+  };
+  f32x16 dk[NDV], dv[NDV];
+#pragma unroll
+  for (int blk = 0; blk < NDV; ++blk)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       dk[blk][i] = 0.f;
       dv[blk][i] = 0.f;
     }
-  for (int q0 = 0; q0 < nq; q0 += kTile) {
-    const int qn = min(kTile, nq - q0);
-    const int t_hi = q0 / a.tq == (q0 + qn - 1) / a.tq ? (q0 + qn - 1) % a.tq : a.tq - 1;
-    if (a.causal_tail && r_first >= tail0 && t_hi < block_min_t) continue;   // uniform over the block
-    __syncthreads();
-    for (int i = threadIdx.x; i < kTile * dim; i += blockDim.x) {
-      const int r = i / dim, d = i - r * dim;
-      const int qr = min(q0 + r, nq - 1);
-      const int hr = g * rep + qr / a.tq, tr = qr % a.tq;
-      const float x = r >= qn ? 0.f
-                      : (d < a.dk ? bf16_to_f32(gp(a.q)[b * a.q_sb + hr * a.q_sh + tr * a.q_st + (d < a.dk ? d : 0)])
-                                  : (d == a.dk ? a.inv_scale_bf16 : 0.f));
-      const uint16_t xb = f32_to_bf16(x);
-      q_t[r * kLdK + d] = xb;
-      if (d < a.dk) qt_t[d * kLdT + r] = xb;
-    }
-    for (int i = threadIdx.x; i < kTile * a.dv; i += blockDim.x) {
-      const int r = i / a.dv, d = i - r * a.dv;
-      const int qr = min(q0 + r, nq - 1);
-      const int hr = g * rep + qr / a.tq, tr = qr % a.tq;
-      const uint16_t x = r >= qn ? 0 : gp(gr.dout)[b * gr.do_sb + hr * gr.do_sh + tr * gr.do_st + d];
-      do_t[r * kLdD + d] = x;
-      dot_t[d * kLdT + r] = x;
-    }
-    for (int i = threadIdx.x; i < kTile * 2; i += blockDim.x) {
-      const int r = i / 2, c = i % 2;
-      st_s[r][c] = r < qn ? stats[(static_cast<int64_t>(lane_ix) * nq + q0 + r) * 2 + c] : 0.f;
-    }
-    __syncthreads();
+  // A query sees this lane's key where its causal index reaches kq.
+  const int kq = a.causal_tail ? key - tail0 : -1;
+  int tile = next_tile(id.split * per), ahead = tile;
+  if (tile < tile_end) {
+    load(tile);
+    store(0);
+    ahead = next_tile(tile + 1);
+    if (ahead < tile_end) load(ahead);
+  }
+  __syncthreads();
+  for (int bf = 0; tile < tile_end; bf ^= 1) {
+    const uint16_t* qt = q_s[bf];
+    const uint16_t* dt = d_s[bf];
     f32x16 s[2], dp[2];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         s[qb][i] = 0.f;
         dp[qb][i] = 0.f;
       }
 #pragma unroll
-      for (int ks = 0; ks < kMaxSteps; ++ks)
-        if (ks < nks)
-          s[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(q_t + (32 * qb + col) * kLdK + 16 * ks + 8 * h),
-                                                          load8(ks_s + (32 * w + col) * kLdK + 16 * ks + 8 * h),
-                                                          s[qb], 0, 0, 0);
-      for (int st = 0; st < nvs; ++st)
-        dp[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(do_t + (32 * qb + col) * kLdD + 16 * st + 8 * h),
-                                                         load8(vs_s + (32 * w + col) * kLdD + 16 * st + 8 * h),
-                                                         dp[qb], 0, 0, 0);
-    }
-    // P and dS of this lane's key against the tile's queries (row i of block qb is query
-    // q0 + 32 qb + 8 (i / 4) + 4 h + i % 4).
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb)
+        s[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(qt + (32 * qb + col) * kLdK + 16 * ks + 8 * h), kf[ks], s[qb], 0, 0, 0);
+#pragma unroll
+    for (int st = 0; st < 2 * NDV; ++st)
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb)
+        dp[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(load8(dt + (32 * qb + col) * kLdD + 16 * st + 8 * h), vf[st], dp[qb], 0, 0, 0);
+    // P and dS of this lane's key against the tile's queries (element i of block qb is query
+    // 32 qb + 8 (i / 4) + 4 h + i % 4).
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int r = 32 * qb + 8 * (i / 4) + 4 * h + (i % 4);
-        const int qr = q0 + r;
-        const int tq_r = qr % a.tq;
-        const bool vis = r < qn && key_ok && !(a.causal_tail && key >= tail0 && key - tail0 > tq_r);
-        const float p = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][i], c2, -st_s[r][0])) : 0.f;
-        s[qb][i] = p;
-        dp[qb][i] = p * (dp[qb][i] - st_s[r][1]);
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int r = 32 * qb + 8 * i4 + 4 * h;
+        const float4 lse = *reinterpret_cast<const float4*>(&lse_s[bf][r]), ds = *reinterpret_cast<const float4*>(&dsum_s[bf][r]);
+        const int4 tt = *reinterpret_cast<const int4*>(&t_s[bf][r]);
+        const float lse4[4] = {lse.x, lse.y, lse.z, lse.w}, ds4[4] = {ds.x, ds.y, ds.z, ds.w};
+        const int t4[4] = {tt.x, tt.y, tt.z, tt.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 4 * i4 + j;
+          const float p = kq <= t4[j] ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][i], c2, -lse4[j])) : 0.f;
+          s[qb][i] = p;
+          dp[qb][i] = p * (dp[qb][i] - ds4[j]);
+        }
       }
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
@@ -399,45 +564,157 @@ __global__ __launch_bounds__(256, 1) void dkv_kernel(logkv_attention_args a, con
       regs_b(s, st, ph, pl);
       regs_b(dp, st, dh, dl);
 #pragma unroll
-      for (int blk = 0; blk < kMaxBlk; ++blk) {
-        if (blk < ndv) {
-          const bf16x8 of = load_t(dot_t, 32 * blk + col, st, h);
-          dv[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of, ph, dv[blk], 0, 0, 0);
-          dv[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of, pl, dv[blk], 0, 0, 0);
-        }
-        if (blk < ndk) {
-          const bf16x8 qf = load_t(qt_t, 32 * blk + col, st, h);
-          dk[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, dh, dk[blk], 0, 0, 0);
-          dk[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, dl, dk[blk], 0, 0, 0);
-        }
+      for (int blk = 0; blk < NDV; ++blk) {
+        const bf16x8 of = load_tr<kLdD>(dt, 32 * blk, st), qf = load_tr<kLdK>(qt, 32 * blk, st);
+        dv[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of, ph, dv[blk], 0, 0, 0);
+        dk[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, dh, dk[blk], 0, 0, 0);
+        dv[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(of, pl, dv[blk], 0, 0, 0);
+        dk[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, dl, dk[blk], 0, 0, 0);
       }
     }
+    tile = ahead;
+    if (tile < tile_end) {
+      store(bf ^ 1);
+      ahead = next_tile(tile + 1);
+      if (ahead < tile_end) load(ahead);
+    }
+    __syncthreads();
   }
-  if (!key_ok || key < first) return;
+  if (!key_ok) return;
+  if (lay.k_splits > 1) {
+    float* out = lay.grad + ((static_cast<int64_t>(lane_ix) * lay.k_splits + id.split) * gr.grad_rows + (key - first)) * (a.dk + a.dv);
+#pragma unroll
+    for (int blk = 0; blk < NDV; ++blk)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const int d = 32 * blk + 8 * i4 + 4 * h, i = 4 * i4;
+        if (d < a.dk) *reinterpret_cast<float4*>(out + d) = make_float4(dk[blk][i], dk[blk][i + 1], dk[blk][i + 2], dk[blk][i + 3]);
+        if (d < a.dv) *reinterpret_cast<float4*>(out + a.dk + d) = make_float4(dv[blk][i], dv[blk][i + 1], dv[blk][i + 2], dv[blk][i + 3]);
+      }
+    return;
+  }
   const int64_t row = static_cast<int64_t>(lane_ix) * gr.grad_rows + (key - first);
 #pragma unroll
-  for (int blk = 0; blk < kMaxBlk; ++blk)
+  for (int blk = 0; blk < NDV; ++blk)
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int d = 32 * blk + 8 * (i / 4) + 4 * h + (i % 4);
-      if (blk < ndk && d < a.dk) gp(gr.dk)[row * a.dk + d] = f32_to_bf16(dk[blk][i] * a.scale);
-      if (blk < ndv && d < a.dv) gp(gr.dv)[row * a.dv + d] = f32_to_bf16(dv[blk][i]);
+      if (d < a.dk) gp(gr.dk)[row * a.dk + d] = f32_to_bf16(dk[blk][i] * a.scale);
+      if (d < a.dv) gp(gr.dv)[row * a.dv + d] = f32_to_bf16(dv[blk][i]);
     }
 }
 
+// dk = scale * and dv = the parts' partials in part order: one thread per row and four features.
+__global__ __launch_bounds__(256) void sum_dkv_kernel(logkv_attention_args a, logkv_attention_grad_args gr, BwdLayout lay) {
+  const int wid = a.dk + a.dv, units = wid / 4;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, lane_ix = blockIdx.y;
+  if (i >= gr.grad_rows * units) return;
+  const int r = i / units, d = 4 * (i % units);
+  const int64_t step = static_cast<int64_t>(gr.grad_rows) * wid;
+  const float* part = lay.grad + static_cast<int64_t>(lane_ix) * lay.k_splits * step + static_cast<int64_t>(r) * wid + d;
+  float x[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int sp = 0; sp < lay.k_splits; ++sp) {
+    const float4 p = *reinterpret_cast<const float4*>(part + sp * step);
+    x[0] += p.x;
+    x[1] += p.y;
+    x[2] += p.z;
+    x[3] += p.w;
+  }
+  const int64_t row = static_cast<int64_t>(lane_ix) * gr.grad_rows + r;
+  const bool key = d < a.dk;
+  LOGKV_G uint16_t* out = key ? gp(gr.dk) + row * a.dk + d : gp(gr.dv) + row * a.dv + (d - a.dk);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) out[j] = f32_to_bf16(key ? x[j] * a.scale : x[j]);
+}
+
+namespace {
+
+// Parts of a walk of `tiles` tiles for `blocks` blocks at one block per CU: the count whose
+// rounds over the 256 CUs cost least, each part charged one tile for its start and partials.
+int bwd_splits(int64_t blocks, int tiles) {
+  int best = 1;
+  double best_cost = 1e30;
+  for (int s = 1; s <= std::min(kMaxSplits, std::max(1, tiles / 2)); ++s) {
+    const double rounds = static_cast<double>((blocks * s + 255) / 256);
+    const double cost = rounds * ((tiles + s - 1) / s + 1) + (s > 1 ? 1 : 0);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  return best;
+}
+
+int dq_splits(const logkv_attention_args& a) {
+  const int nq = a.n_heads / a.n_groups * a.tq;
+  return bwd_splits(static_cast<int64_t>((nq + kQRows - 1) / kQRows) * a.n_batch * a.n_groups, (a.cap + kTile - 1) / kTile);
+}
+
+int dkv_splits(const logkv_attention_args& a, int grad_rows) {
+  const int nq = a.n_heads / a.n_groups * a.tq;
+  return bwd_splits(static_cast<int64_t>((grad_rows + kKRows - 1) / kKRows) * a.n_batch * a.n_groups, (nq + kTile - 1) / kTile);
+}
+
+// Workspace floats: [stats][parts][gradient partials], the last for dq and for the dk / dv of a
+// chunk (grad_rows = tq); more gradient rows take as many parts as fit it.
+struct BwdSizes {
+  int64_t stats, part, grad;
+};
+BwdSizes bwd_sizes(const logkv_attention_args& a) {
+  const int nq = a.n_heads / a.n_groups * a.tq, qs = dq_splits(a), ks = dkv_splits(a, a.tq);
+  const int64_t lanes = static_cast<int64_t>(a.n_batch) * a.n_groups;
+  const int64_t dq = qs > 1 ? lanes * qs * nq * a.dk : 0, dkv = ks > 1 ? lanes * ks * a.tq * (a.dk + a.dv) : 0;
+  return {(lanes * nq * 2 + 3) / 4 * 4, lanes * qs * nq * 4, std::max(dq, dkv)};
+}
+
+bool aligned(const void* p, int64_t sb, int64_t sh, int64_t st, int bytes) {
+  const int64_t n = bytes / 2;
+  return reinterpret_cast<uintptr_t>(p) % bytes == 0 && sb % n == 0 && sh % n == 0 && st % n == 0;
+}
+
+}  // namespace
+
 int64_t chunk_backward_workspace_floats(const logkv_attention_args& a) {
-  const int nq = (a.n_heads / a.n_groups) * a.tq;
-  return static_cast<int64_t>(a.n_batch) * a.n_groups * nq * 2;
+  const BwdSizes z = bwd_sizes(a);
+  return z.stats + z.part + z.grad;
 }
 
 int launch_chunk_backward(const logkv_attention_args& a, const int32_t* width, const logkv_attention_grad_args& g,
-                          float* stats, hipStream_t stream) {
+                          float* ws, hipStream_t stream) {
   const int nq = (a.n_heads / a.n_groups) * a.tq;
   const int lanes = a.n_batch * a.n_groups;
-  hipLaunchKernelGGL(dq_kernel, dim3((nq + kRows - 1) / kRows, lanes), dim3(256), 0, stream, a, width, g, stats);
-  if (g.grad_rows > 0)
-    hipLaunchKernelGGL(dkv_kernel, dim3((g.grad_rows + kRows - 1) / kRows, lanes), dim3(256), 0, stream, a, width, g,
-                       stats);
+  const BwdSizes z = bwd_sizes(a);
+  BwdLayout lay{};
+  lay.q_splits = dq_splits(a);
+  lay.k_splits = 1;
+  if (g.grad_rows > 0) {
+    const int64_t fit = z.grad / (static_cast<int64_t>(lanes) * g.grad_rows * (a.dk + a.dv));
+    lay.k_splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(dkv_splits(a, g.grad_rows), fit)));
+  }
+  lay.vec_q = aligned(a.q, a.q_sb, a.q_sh, a.q_st, 16);
+  lay.vec_do = aligned(g.dout, g.do_sb, g.do_sh, g.do_st, 16);
+  lay.vec_dq = aligned(g.dq, g.dq_sb, g.dq_sh, g.dq_st, 8);
+  lay.stats = ws;
+  lay.part = ws + z.stats;
+  lay.grad = ws + z.stats + z.part;
+  const dim3 qgrid((nq + kQRows - 1) / kQRows, lay.q_splits, lanes);
+  const dim3 kgrid((g.grad_rows + kKRows - 1) / kKRows, lay.k_splits, lanes);
+  auto run = [&](auto stats, auto dq, auto dkv) {
+    hipLaunchKernelGGL(stats, qgrid, dim3(64 * kQWaves), 0, stream, a, width, g, lay);
+    hipLaunchKernelGGL(dq, qgrid, dim3(64 * kQWaves), 0, stream, a, width, g, lay);
+    if (lay.q_splits > 1)
+      hipLaunchKernelGGL(sum_dq_kernel, dim3((nq * (a.dk / 4) + 255) / 256, lanes), dim3(256), 0, stream, a, g, lay);
+    if (g.grad_rows > 0) {
+      hipLaunchKernelGGL(dkv, kgrid, dim3(64 * kKWaves), 0, stream, a, width, g, lay);
+      if (lay.k_splits > 1)
+        hipLaunchKernelGGL(sum_dkv_kernel, dim3((static_cast<unsigned>(g.grad_rows) * ((a.dk + a.dv) / 4) + 255) / 256, lanes),
+                           dim3(256), 0, stream, a, g, lay);
+    }
+  };
+  // Head dim 64 (5 steps of the packed width, 2 blocks of dk and dv) has its own kernels; every
+  // other shape runs the full ones on zero padding.
+  if (a.dim <= 80 && a.dk <= 64 && a.dv <= 64) run(stats_kernel<5, 2>, dq_kernel<5, 2>, dkv_kernel<5, 2>);
+  else run(stats_kernel<9, 4>, dq_kernel<9, 4>, dkv_kernel<9, 4>);
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }
 
