@@ -783,12 +783,12 @@ def decode_workload(args, torch, np):
         "device_ms_per_token_note": "one step's pack + attention, 8 steps captured back to back in a HIP graph and "
                                     "replayed 8 times (no host work)",
         "packed_rows_per_lane": rows, "pooled_width": width,
-        "roofline": {"kernel": "stream_kernel + combine_kernel", "bound": "hbm", "achieved": achieved,
+        "roofline": {"kernel": "decode_mfma_kernel + combine_kernel", "bound": "hbm", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "algorithmic_bytes_per_launch": attn_bytes, "bytes_per_packed_row": row_bytes,
                      "avg_launch_ms": attn_ms,
                      "timing": "HIP events around 8 replays of a HIP graph holding 8 back-to-back attention calls "
-                               "(stream_kernel + combine_kernel each)"},
+                               "(decode_mfma_kernel + combine_kernel each)"},
     }
 
 

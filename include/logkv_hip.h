@@ -551,7 +551,7 @@ int logkv_chunk_attention(const logkv_attention_args* args, const int32_t* table
  * training block, or every slot), dk [n_batch, G, grad_rows, dk] and dv
  * [n_batch, G, grad_rows, dv] (bf16, contiguous). grad_rows <= tail. dk a multiple
  * of 8 up to 128, dv in {32, 64, 96, 128}, packed width up to 144. The workspace
- * (logkv_chunk_backward_workspace_bytes, 16-byte aligned) holds each query's
+ * (logkv_chunk_backward_workspace_bytes) holds each query's
  * log-sum-exp and dout . out and the partials of the split ranges between the
  * launches.
  * Replaces the autograd backward of the Flash SDPA call on the packed workspace

@@ -804,8 +804,6 @@ int logkv_chunk_attention_backward(const logkv_attention_args* a, const int32_t*
     return fail(LOGKV_EINVAL, "packed K/V must be 16-byte aligned");
   if (!ws || ws_bytes < logkv::chunk_backward_workspace_floats(*a) * 4)
     return fail(LOGKV_EINVAL, "attention backward workspace too small");
-  if (reinterpret_cast<uintptr_t>(ws) % 16)
-    return fail(LOGKV_EINVAL, "attention backward workspace must be 16-byte aligned");
   const int rc = logkv::launch_chunk_backward(*a, table + table_ints - 1, *gr, static_cast<float*>(ws),
                                               static_cast<hipStream_t>(stream));
   if (rc) return launch_failed(rc, "attention backward");

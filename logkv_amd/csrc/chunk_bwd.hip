@@ -478,9 +478,9 @@ __global__ __launch_bounds__(64 * kKWaves, 1) void dkv_kernel(logkv_attention_ar
     if (tid < kTile) {
       const int qr = min(q0 + tid, nq - 1);
       const float2 x = *reinterpret_cast<const float2*>(lay.stats + (static_cast<int64_t>(lane_ix) * nq + qr) * 2);
-      lse_x = q0 + tid < nq ? x.x : __builtin_inff();   // rows past the queries: p = 2^(-inf) = 0
+      lse_x = x.x;
       dsum_x = x.y;
-      t_x = qr % a.tq;
+      t_x = q0 + tid < nq ? qr % a.tq : INT32_MIN;   // rows past the queries see no key: p = 0
     }
   };
   auto store = [&](int bf) {
@@ -676,7 +676,7 @@ bool aligned(const void* p, int64_t sb, int64_t sh, int64_t st, int bytes) {
 
 int64_t chunk_backward_workspace_floats(const logkv_attention_args& a) {
   const BwdSizes z = bwd_sizes(a);
-  return z.stats + z.part + z.grad;
+  return z.stats + z.part + z.grad + 3;   // the regions start at the workspace's first 16-byte boundary
 }
 
 int launch_chunk_backward(const logkv_attention_args& a, const int32_t* width, const logkv_attention_grad_args& g,
@@ -694,9 +694,9 @@ int launch_chunk_backward(const logkv_attention_args& a, const int32_t* width, c
   lay.vec_q = aligned(a.q, a.q_sb, a.q_sh, a.q_st, 16);
   lay.vec_do = aligned(g.dout, g.do_sb, g.do_sh, g.do_st, 16);
   lay.vec_dq = aligned(g.dq, g.dq_sb, g.dq_sh, g.dq_st, 8);
-  lay.stats = ws;
-  lay.part = ws + z.stats;
-  lay.grad = ws + z.stats + z.part;
+  lay.stats = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(ws) + 15) / 16 * 16);
+  lay.part = lay.stats + z.stats;
+  lay.grad = lay.part + z.part;
   const dim3 qgrid((nq + kQRows - 1) / kQRows, lay.q_splits, lanes);
   const dim3 kgrid((g.grad_rows + kKRows - 1) / kKRows, lay.k_splits, lanes);
   auto run = [&](auto stats, auto dq, auto dkv) {

@@ -15,9 +15,8 @@
 // Decode attention (litgpt/log_kv_cache.py:6428-6464, :6751-6758):
 // softmax(scale * [q, 1/scale] . [k, bias]) v over the packed rows, the last
 // `causal_tail` rows causal against the queries, query head h reading KV group
-// h / (Hq / G). Flash-decoding: row splits per lane, each staging 64-row K and
-// V tiles in LDS with an online softmax; a second kernel combines the splits in
-// a fixed order.
+// h / (Hq / G). Flash-decoding: row splits per lane (decode_mfma.hip), combined
+// here by a second kernel in a fixed order.
 #include <algorithm>
 #include <type_traits>
 
@@ -27,16 +26,7 @@ namespace logkv {
 
 namespace {
 
-typedef __bf16 rd_bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int kPlanThreads = 1024;
-constexpr int kTile = 64;          // rows per staged K/V tile
-constexpr int kSplitRows = 512;    // rows per attention split (staged decode kernel)
-constexpr int kStreamRows = 512;   // most rows per split of the streaming kernel when the grid is not the limit
-constexpr int kStreamBlocks = 640;    // streaming blocks per launch at most: 2.5 per CU, so splits are long enough to
-                                      // amortize a block's start and end (1280 / 1024 / 512 / 320 measured slower)
-constexpr int kMaxQ = 16;          // queries per KV group (heads per group x query rows)
-constexpr int kMaxPacked = 264;    // packed row width limit (dk + 1 rounded to 8, dv)
-constexpr int kAccPerThread = kMaxQ * kMaxDim / 256;   // outputs per thread of a 256-thread split block
 
 struct PlanCtx {
   const LOGKV_G int16_t* count;    // [lanes, K, L]
@@ -375,282 +365,6 @@ __global__ __launch_bounds__(256) void pack_kernel(logkv_readout_view c, logkv_p
   }
 }
 
-// Split attention: partial (max, sum, acc) per (split, lane, query).
-__global__ __launch_bounds__(256) void decode_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
-                                                     float* __restrict__ part) {
-  __shared__ float q_s[kMaxQ * kMaxPacked];
-  __shared__ __align__(16) uint16_t kv_s[kTile * kMaxPacked];
-  __shared__ float p_s[kMaxQ * kTile];
-  __shared__ float m_s[kMaxQ], l_s[kMaxQ], corr_s[kMaxQ];
-  const int lane = blockIdx.y;
-  const int G = a.n_groups;
-  const int b = lane / G, g = lane % G;
-  const int rep = a.n_heads / G;
-  const int nq = rep * a.tq;
-  const int dim = a.dim;
-  const int total = min(*width_ptr + a.tail + (a.alpha_count_dev ? *a.alpha_count_dev : 0), a.cap);
-  const int r_begin = blockIdx.x * kSplitRows;
-  const int r_end = min(r_begin + kSplitRows, total);
-  float* out = part + (static_cast<int64_t>(lane) * gridDim.x + blockIdx.x) * nq * (a.dv + 2);
-  // Queries [q, 1/scale (bf16), 0...] as float; query qi = head (g*rep + qi / tq), row qi % tq.
-  for (int i = threadIdx.x; i < nq * dim; i += blockDim.x) {
-    const int qi = i / dim, d = i % dim;
-    const int h = g * rep + qi / a.tq, t = qi % a.tq;
-    float x = 0.f;
-    if (d < a.dk) x = bf16_to_f32(gp(a.q)[b * a.q_sb + h * a.q_sh + t * a.q_st + d]);
-    else if (d == a.dk) x = a.inv_scale_bf16;
-    q_s[qi * kMaxPacked + d] = x;
-  }
-  for (int qi = threadIdx.x; qi < nq; qi += blockDim.x) {
-    m_s[qi] = -__builtin_inff();
-    l_s[qi] = 0.f;
-  }
-  const int w = wave_id(), l = lane_id(), nw = blockDim.x / kWave;
-  float acc[kAccPerThread];
-#pragma unroll
-  for (int i = 0; i < kAccPerThread; ++i) acc[i] = 0.f;
-  const int n_out = nq * a.dv;
-  const int per = (n_out + blockDim.x - 1) / blockDim.x;
-  const LOGKV_G uint16_t* kbase = gp(a.k) + static_cast<int64_t>(lane) * a.cap * dim;
-  const LOGKV_G uint16_t* vbase = gp(a.v) + static_cast<int64_t>(lane) * a.cap * dim;
-  const int units = dim / 8;   // 16-byte units per packed row
-  const int tail0 = total - a.causal_tail;
-  for (int t0 = r_begin; t0 < r_end; t0 += kTile) {
-    const int rows = min(kTile, r_end - t0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < rows * units; i += blockDim.x) {
-      const int r = i / units, u = i % units;
-      *reinterpret_cast<uint4*>(kv_s + r * dim + 8 * u) =
-          *(const LOGKV_G uint4*)(kbase + (static_cast<int64_t>(t0) + r) * dim + 8 * u);
-    }
-    __syncthreads();
-    // Scores and online softmax: the wave owning query qi has one row per lane.
-    for (int qi = w; qi < nq; qi += nw) {
-      const int r = l;
-      float sc = -__builtin_inff();
-      if (r < rows) {
-        float dot = 0.f;
-        const float* qv = q_s + qi * kMaxPacked;
-        const uint16_t* kr = kv_s + r * dim;
-        for (int d = 0; d < dim; d += 2) {
-          const uint32_t pair = *reinterpret_cast<const uint32_t*>(kr + d);
-          dot = __builtin_fmaf(qv[d], __uint_as_float(pair << 16), dot);
-          dot = __builtin_fmaf(qv[d + 1], __uint_as_float(pair & 0xffff0000u), dot);
-        }
-        sc = a.scale * dot;
-        const int row = t0 + r;
-        if (a.causal_tail && row >= tail0 && row - tail0 > qi % a.tq) sc = -__builtin_inff();
-      }
-      float mx = sc;
-      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-      const float m_old = m_s[qi];
-      const float m_new = fmaxf(m_old, mx);
-      const float corr = m_new == -__builtin_inff() ? 1.f : __expf(m_old - m_new);
-      const float pr = sc == -__builtin_inff() ? 0.f : __expf(sc - m_new);
-      float sum = pr;
-      for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, kWave);
-      p_s[qi * kTile + r] = pr;
-      if (l == 0) {
-        l_s[qi] = l_s[qi] * corr + sum;
-        m_s[qi] = m_new;
-        corr_s[qi] = corr;
-      }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < rows * units; i += blockDim.x) {
-      const int r = i / units, u = i % units;
-      *reinterpret_cast<uint4*>(kv_s + r * dim + 8 * u) =
-          *(const LOGKV_G uint4*)(vbase + (static_cast<int64_t>(t0) + r) * dim + 8 * u);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kAccPerThread; ++k) {
-      const int o = threadIdx.x + k * blockDim.x;
-      if (k < per && o < n_out) {
-        const int qi = o / a.dv, d = o % a.dv;
-        float s = acc[k] * corr_s[qi];
-        const float* pq = p_s + qi * kTile;
-        for (int r = 0; r < rows; ++r) s = __builtin_fmaf(pq[r], bf16_to_f32(kv_s[r * dim + d]), s);
-        acc[k] = s;
-      }
-    }
-  }
-  __syncthreads();
-  // Partials: [m, l, acc[dv]] per query.
-  for (int qi = threadIdx.x; qi < nq; qi += blockDim.x) {
-    out[qi * (a.dv + 2)] = m_s[qi];
-    out[qi * (a.dv + 2) + 1] = l_s[qi];
-  }
-#pragma unroll
-  for (int k = 0; k < kAccPerThread; ++k) {
-    const int o = threadIdx.x + k * blockDim.x;
-    if (k < per && o < n_out) out[(o / a.dv) * (a.dv + 2) + 2 + o % a.dv] = acc[k];
-  }
-}
-
-// Streaming decode for at most 4 queries per KV group (a decode step of GQA
-// heads): no staging of K / V in LDS. A block is 16 row groups of 16 lanes; a
-// group reads one packed row at a time (its 16-byte units spread over the 16
-// lanes: [q, 1/scale] . [k, bias] folded over the group), keeps its own online
-// softmax per query and accumulates its lanes' 8-wide slices of V, rows
-// 4 at a time with all loads issued first; 512-row splits. At the end of the split the 16
-// groups are combined in LDS in group order and the split's partials go to
-// the workspace in the layout the split combine reads.
-//
-// SPLIT (dk a multiple of 8): the key's bias column dk starts a unit of its
-// own, so the 16-byte units cover only the dk features and the bias is one
-// 2-byte load per row, added after the group fold as q[dk] * bias; UJ then
-// counts units of the dk features only (8 registers per row and query fewer).
-template <int NQ, int UJ, bool SPLIT>
-__global__ __launch_bounds__(256) void stream_kernel(logkv_attention_args a, const int32_t* __restrict__ width_ptr,
-                                                     float* __restrict__ part) {
-  constexpr int kGroups = 16, kGl = 16, kRows = 4;
-  __shared__ float m_s[kGroups][NQ], l_s[kGroups][NQ];
-  __shared__ float acc_s[kGroups][NQ][128];
-  const int lane = blockIdx.y, G = a.n_groups;
-  const int b = lane / G, g = lane % G;
-  const int rep = a.n_heads / G, nq = rep * a.tq;
-  const int grp = threadIdx.x / kGl, gl = threadIdx.x % kGl;
-  const int dim = a.dim, units = SPLIT ? a.dk / 8 : dim / 8, vunits = (a.dv + 7) / 8;   // the last unit may run into the zero pad (dim >= 8 * vunits)
-  const float q_bias = a.inv_scale_bf16;
-  const int total = min(*width_ptr + a.tail + (a.alpha_count_dev ? *a.alpha_count_dev : 0), a.cap);
-  const int tail0 = total - a.causal_tail;
-  // The lane's rows in gridDim.x equal shares, multiples of 64 (a pass of the
-  // 16 row groups x 4 rows); splits past the rows write empty partials.
-  const int share = max(64, (total + 64 * static_cast<int>(gridDim.x) - 1) / (64 * static_cast<int>(gridDim.x)) * 64);
-  const int r_begin = blockIdx.x * share, r_end = min(r_begin + share, total);
-  float* out = part + (static_cast<int64_t>(lane) * gridDim.x + blockIdx.x) * nq * (a.dv + 2);
-  // This lane's slices of the queries [q, 1/scale (bf16), 0...]: units gl + 16 j,
-  // as bf16 pairs (features 2e, 2e + 1 of a unit) for the packed dot products.
-  uint32_t qp[NQ][UJ][4];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int qq = q < nq ? q : nq - 1;
-    const int h = g * rep + qq / a.tq, t = qq % a.tq;
-#pragma unroll
-    for (int j = 0; j < UJ; ++j) {
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        uint32_t pair = 0u;
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const int d = 8 * (gl + kGl * j) + e + hf;
-          uint32_t x = 0u;
-          if (d < a.dk) x = gp(a.q)[b * a.q_sb + h * a.q_sh + t * a.q_st + d];
-          else if (!SPLIT && d == a.dk) x = f32_to_bf16(a.inv_scale_bf16);
-          pair |= (q < nq ? x : 0u) << (16 * hf);
-        }
-        qp[q][j][e / 2] = pair;
-      }
-    }
-  }
-  float m[NQ], l[NQ], acc[NQ][8];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    m[q] = -__builtin_inff();
-    l[q] = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[q][e] = 0.f;
-  }
-  const LOGKV_G uint16_t* kbase = gp(a.k) + static_cast<int64_t>(lane) * a.cap * dim;
-  const LOGKV_G uint16_t* vbase = gp(a.v) + static_cast<int64_t>(lane) * a.cap * dim;
-  const bool v_on = gl < vunits;
-  for (int r0 = r_begin + grp; r0 < r_end; r0 += kGroups * kRows) {
-    uint4 kx[kRows][UJ], vx[kRows];
-    uint16_t kb[kRows];
-#pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-      const int row = min(r0 + kGroups * i, r_end - 1);
-#pragma unroll
-      for (int j = 0; j < UJ; ++j) {
-        const int u = min(gl + kGl * j, units - 1);
-        kx[i][j] = *(const LOGKV_G uint4*)(kbase + static_cast<int64_t>(row) * dim + 8 * u);
-      }
-      if (SPLIT) kb[i] = kbase[static_cast<int64_t>(row) * dim + a.dk];
-      vx[i] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(row) * dim + 8 * (v_on ? gl : 0));
-    }
-#pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-      const int row = r0 + kGroups * i;
-      if (row >= r_end) break;
-      float dot[NQ];
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) dot[q] = 0.f;
-#pragma unroll
-      for (int j = 0; j < UJ; ++j) {
-        if (gl + kGl * j < units) {
-          const uint32_t w4[4] = {kx[i][j].x, kx[i][j].y, kx[i][j].z, kx[i][j].w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-#pragma unroll
-            for (int q = 0; q < NQ; ++q)
-              dot[q] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(rd_bf16x2, w4[e]),
-                                                       __builtin_bit_cast(rd_bf16x2, qp[q][j][e]), dot[q], false);
-          }
-        }
-      }
-      const uint32_t v4[4] = {vx[i].x, vx[i].y, vx[i].z, vx[i].w};
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-#pragma unroll
-        for (int off = kGl / 2; off >= 1; off >>= 1) dot[q] += __shfl_xor(dot[q], off, kGl);
-        if (SPLIT) dot[q] = __builtin_fmaf(q_bias, bf16_to_f32(kb[i]), dot[q]);
-        float sc = a.scale * dot[q];
-        const int t = (q < nq ? q : nq - 1) % a.tq;
-        if (q >= nq || (a.causal_tail && row >= tail0 && row - tail0 > t)) sc = -__builtin_inff();
-        const float m_new = fmaxf(m[q], sc);
-        const float p = sc == -__builtin_inff() ? 0.f : __expf(sc - m_new);
-        // A new maximum rescales the sums; otherwise the factor is exactly 1
-        // (2^0) and the products by it change nothing, so a wave whose lanes
-        // all kept their maximum skips them.
-        if (__ballot(m_new != m[q])) {
-          const float corr = m_new == -__builtin_inff() ? 1.f : __expf(m[q] - m_new);
-          l[q] = l[q] * corr;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[q][e] = acc[q][e] * corr;
-        }
-        l[q] = l[q] + p;
-        m[q] = m_new;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[q][2 * e] = __builtin_fmaf(p, __uint_as_float(v4[e] << 16), acc[q][2 * e]);
-          acc[q][2 * e + 1] = __builtin_fmaf(p, __uint_as_float(v4[e] & 0xffff0000u), acc[q][2 * e + 1]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    if (gl == 0) {
-      m_s[grp][q] = m[q];
-      l_s[grp][q] = l[q];
-    }
-    if (v_on) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc_s[grp][q][8 * gl + e] = acc[q][e];
-    }
-  }
-  __syncthreads();
-  // Groups combined in group order: [m, l, acc[dv]] per query of this split.
-  for (int o = threadIdx.x; o < nq * (a.dv + 2); o += blockDim.x) {
-    const int q = o / (a.dv + 2), c = o % (a.dv + 2);
-    float mx = -__builtin_inff();
-    for (int gg = 0; gg < kGroups; ++gg) mx = fmaxf(mx, m_s[gg][q]);
-    float val;
-    if (c == 0) {
-      val = mx;
-    } else {
-      val = 0.f;
-      for (int gg = 0; gg < kGroups; ++gg) {
-        if (m_s[gg][q] == -__builtin_inff()) continue;
-        const float f = __expf(m_s[gg][q] - mx);
-        val += (c == 1 ? l_s[gg][q] : acc_s[gg][q][c - 2]) * f;
-      }
-    }
-    out[o] = val;
-  }
-}
-
 // Combine the splits of each (lane, query) in split order: one block per
 // (lane, query), one output feature per thread. An empty split carries
 // m = -inf with zero sums, so it adds exp(-inf) * 0 = 0 and needs no test.
@@ -762,30 +476,21 @@ int launch_pack(const logkv_readout_view& c, const logkv_pack_args& p, const int
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }
 
-// 16-byte key units per row group lane of the streaming kernel (the bias
-// column excluded when it starts a unit of its own).
-int stream_key_units(const logkv_attention_args& a) {
-  const int units = a.dk % 8 == 0 ? a.dk / 8 : a.dim / 8;
-  return (units + 15) / 16;
-}
-
-bool use_stream(const logkv_attention_args& a) {
-  const int nq = (a.n_heads / a.n_groups) * a.tq;
-  return nq <= 4 && a.dv <= 128 && a.dk >= 8 && stream_key_units(a) <= 3;
-}
-
-// Splits per lane: the staged kernel takes kSplitRows rows each; the streaming
-// kernel takes up to kStreamRows each, but no more splits than keep every block
-// of the launch resident at once (its splits then share the rows equally).
+// Splits per lane: at most one per 128 rows (a 32-row tile for each of a block's four waves), and
+// no more than keep every block of the launch resident (two per CU; one for packed widths above
+// 160). 64 lanes of 8.4K rows of 128 features: 51 us at 512 blocks, 58 at 768, 57 at 1024.
 int attention_splits(const logkv_attention_args& a) {
-  if (!use_stream(a)) return (a.cap + kSplitRows - 1) / kSplitRows;
-  const int lanes = a.n_batch * a.n_groups;
-  return std::max(1, std::min((a.cap + kStreamRows - 1) / kStreamRows, kStreamBlocks / std::max(1, lanes)));
+  const int lanes = a.n_batch * a.n_groups, blocks = a.dim <= 160 && a.dv <= 128 ? 512 : 256;
+  return std::max(1, std::min((a.cap + 127) / 128, blocks / std::max(1, lanes)));
 }
 
+// Partials of the launch, or for more than 4 queries or dv > 128 room for one per 512 rows of
+// capacity when that is more: the size (and with it what fits the static scratch) that callers
+// of those shapes were always asked for.
 int64_t attention_workspace_floats(const logkv_attention_args& a) {
-  const int n_split = attention_splits(a);
   const int nq = (a.n_heads / a.n_groups) * a.tq;
+  const bool few = nq <= 4 && a.dv <= 128 && a.dk >= 8;
+  const int n_split = std::max(attention_splits(a), few ? 1 : (a.cap + 511) / 512);
   return static_cast<int64_t>(a.n_batch) * a.n_groups * n_split * nq * (a.dv + 2);
 }
 
@@ -797,33 +502,8 @@ int launch_combine(const logkv_attention_args& a, const float* part, int n_split
 
 int launch_attention(const logkv_attention_args& a, const int32_t* width, float* part, hipStream_t stream) {
   const int n_split = attention_splits(a);
-  const int lanes = a.n_batch * a.n_groups;
-  const int nq = (a.n_heads / a.n_groups) * a.tq;
-  const int uj = stream_key_units(a);
-  const dim3 grid(n_split, lanes);
-  auto stream_launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, width, part);
-  };
-  auto by_units = [&](auto one, auto two, auto three) {
-    if (uj == 1) stream_launch(one);
-    else if (uj == 2) stream_launch(two);
-    else stream_launch(three);
-  };
-  if (use_stream(a)) {
-    if (a.dk % 8 == 0) {
-      if (nq == 1) by_units(stream_kernel<1, 1, true>, stream_kernel<1, 2, true>, stream_kernel<1, 3, true>);
-      else if (nq == 2) by_units(stream_kernel<2, 1, true>, stream_kernel<2, 2, true>, stream_kernel<2, 3, true>);
-      else by_units(stream_kernel<4, 1, true>, stream_kernel<4, 2, true>, stream_kernel<4, 3, true>);
-    } else {
-      if (nq == 1) by_units(stream_kernel<1, 1, false>, stream_kernel<1, 2, false>, stream_kernel<1, 3, false>);
-      else if (nq == 2) by_units(stream_kernel<2, 1, false>, stream_kernel<2, 2, false>, stream_kernel<2, 3, false>);
-      else by_units(stream_kernel<4, 1, false>, stream_kernel<4, 2, false>, stream_kernel<4, 3, false>);
-    }
-  } else {
-    hipLaunchKernelGGL(decode_kernel, grid, dim3(256), 0, stream, a, width, part);
-  }
-  hipLaunchKernelGGL(combine_kernel, dim3(lanes, nq), dim3(a.dv <= 64 ? 64 : 128), 0, stream, a, part, n_split);
-  return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
+  const int rc = launch_decode_mfma(a, width, part, n_split, stream);
+  return rc ? rc : launch_combine(a, part, n_split, stream);
 }
 
 }  // namespace logkv
