@@ -74,7 +74,7 @@ int check_rows(const logkv_ladder_view* c, const logkv_rows_view* r) {
 }
 
 struct Plan {
-  int64_t order, assign, s_win, dist, snap, plans, tok, units, ladder, total;
+  int64_t order, assign, s_win, snap, plans, tok, units, ladder, total;
   int64_t stride, s0, m0;
   int32_t sort_width;
 };
@@ -95,8 +95,6 @@ Plan plan_for(const logkv_ladder_view* c, int32_t tokens, int32_t late, int32_t 
   p.assign = off;
   off += align256(lanes * tokens);
   p.s_win = off;
-  off += align256(lanes * tokens * 4);
-  p.dist = off;
   off += align256(lanes * tokens * 4);
   p.snap = off;
   off += align256(ladders);
@@ -139,7 +137,6 @@ int carve(const logkv_ladder_view* c, const logkv_rows_view* r, const logkv_rout
   ws.order = order ? order : reinterpret_cast<int32_t*>(base + p.order);
   ws.assign = assign ? assign : reinterpret_cast<int8_t*>(base + p.assign);
   ws.s_win = reinterpret_cast<float*>(base + p.s_win);
-  ws.dist = reinterpret_cast<float*>(base + p.dist);
   ws.snap_alive = base + p.snap;
   ws.ladder = base + p.ladder;
   ws.cap_dist = reinterpret_cast<float*>(base + p.ladder);

@@ -618,21 +618,6 @@ __global__ __launch_bounds__(kAttachMfmaWaves* kWave) void attach_mfma_kernel(
   }
 }
 
-// Canonical squared distance between a row (held in x[]) and another bf16 row.
-__device__ __forceinline__ float row_d2_bf16(const float* x, const uint16_t* other, int D, int J) {
-  const int l = lane_id();
-  float s = 0.f;
-#pragma unroll
-  for (int j = 0; j < kMaxDim / kWave; ++j) {
-    if (j < J) {
-      const int d = l + j * kWave;
-      const float diff = d < D ? x[j] - bf16_to_f32(other[d]) : 0.f;
-      s = j == 0 ? diff * diff : s + diff * diff;
-    }
-  }
-  return wave_sum0(s);
-}
-
 // Block-wide argmax (first index on ties) of (value, index) pairs.
 __device__ __forceinline__ void block_argmax(float& v, int& i, float* sv, int* si) {
   for (int off = 32; off >= 1; off >>= 1) {
@@ -669,6 +654,80 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
 }
 
 // ---------------------------------------------------------------------------
+// Canonical squared distances of 8 rows per wave: a group of 8 lanes takes a
+// row, lane c of the group the 8 features of 16-byte unit u(c) of each 64-wide
+// slice (leaves 8 u .. 8 u + 7 of the canonical sum). The halving tree's folds
+// over leaves l and l + 32, + 16, + 8 are exchanges with the lanes holding
+// units u ^ 4, u ^ 2, u ^ 1 (each keeps half of its values), which leaves leaf
+// u in the lane; the folds + 4, + 2, + 1 use the same three exchanges. u is
+// chosen so that these are the DPP patterns lane ^ 7, ^ 2 and ^ 1. Sums are
+// those of wave_sum0, at 80 vector instructions per 8 rows instead of 25 a row.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int group_unit() {
+  const int c = lane_id() & 7;
+  return (c & 3) ^ ((c & 4) ? 7 : 0);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+
+constexpr int kLaneXor7 = 0x141, kLaneXor2 = 0x4E, kLaneXor1 = 0xB1;   // row_half_mirror, quad_perm [2,3,0,1] / [1,0,3,2]
+
+__device__ __forceinline__ float group_fold(const float (&e)[8], int u) {
+  float f[4], g[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = ((u & 4) ? e[4 + i] : e[i]) + dpp_f32<kLaneXor7>((u & 4) ? e[i] : e[4 + i]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) g[i] = ((u & 2) ? f[2 + i] : f[i]) + dpp_f32<kLaneXor2>((u & 2) ? f[i] : f[2 + i]);
+  float s = ((u & 1) ? g[1] : g[0]) + dpp_f32<kLaneXor1>((u & 1) ? g[0] : g[1]);
+  s = s + dpp_f32<kLaneXor7>(s);
+  s = s + dpp_f32<kLaneXor2>(s);
+  return s + dpp_f32<kLaneXor1>(s);
+}
+
+// The lane's units of a row of J 64-wide slices (features past D zero).
+template <int J>
+__device__ __forceinline__ void load_units(const LOGKV_G uint16_t* row, int u, int D, bool vec, uint4 (&x)[J]) {
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int d = 64 * j + 8 * u;
+    if (vec) {
+      x[j] = *(const LOGKV_G uint4*)(row + (d < D ? d : 0));
+      if (d >= D) x[j] = make_uint4(0, 0, 0, 0);
+    } else {
+      uint32_t e[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        e[i] = row[d + i < D ? d + i : D - 1];
+        if (d + i >= D) e[i] = 0u;
+      }
+      x[j] = make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
+    }
+  }
+}
+
+template <int J>
+__device__ __forceinline__ float unit_feature(const uint4 (&x)[J], int j, int i) {
+  const uint32_t w4[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+  return __uint_as_float((i & 1) ? w4[i / 2] & 0xffff0000u : w4[i / 2] << 16);
+}
+
+template <int J>
+__device__ __forceinline__ float group_d2(const uint4 (&x)[J], const float (&p)[J][8], int u) {
+  float e[8];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float diff = unit_feature<J>(x, j, i) - p[j][i];
+      e[i] = j == 0 ? diff * diff : e[i] + diff * diff;
+    }
+  return group_fold(e, u);
+}
+
+// ---------------------------------------------------------------------------
 // Seeds for lanes with free cluster slots (one block per lane), then the
 // orphans' clusters.
 //
@@ -680,13 +739,22 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
 // rows it already took: its kept direct rows, or 1 for a seeded slot), or the
 // nearest candidate when none has room. The distances go to `cap_dist` in
 // orphan order, then one wave walks them in chunks staged through LDS.
+//
+// Bound by the vector instructions of the squared distances (one block per
+// lane): 11 farthest-point passes over 2048 rows of 128 features, the nearest
+// seed kept along the way so that assigning the orphans takes one more, 0.19 ms
+// against 1.1 ms with a row per wave and a second round over all candidates.
+// J 64-wide slices of the features.
 // ---------------------------------------------------------------------------
-template <bool CAPPED>
+template <bool CAPPED, int J>
 __global__ __launch_bounds__(1024) void seed_kernel(LadderArgs c, RowsArgs r, RouteParams prm,
                                                     const int32_t* __restrict__ order, int8_t* __restrict__ assign,
-                                                    const float* __restrict__ s_win, float* __restrict__ dist,
+                                                    const float* __restrict__ s_win,
                                                     float* __restrict__ cap_dist) {
-  __shared__ float cand_s[kMaxClusters * kMaxDim];
+  __shared__ float ds_l[kMaxOrderRows];        // running distance of a row to the nearest seed
+  __shared__ uint16_t ord_l[kMaxOrderRows];    // row offset of a position-order index
+  __shared__ int8_t arg_l[CAPPED ? 1 : kMaxOrderRows];   // cluster of the nearest seed
+  __shared__ __align__(16) float cand_s[kMaxClusters * kMaxDim];
   __shared__ float red_v[16];
   __shared__ int red_i[16];
   __shared__ int picks_s[kMaxClusters];
@@ -697,7 +765,7 @@ __global__ __launch_bounds__(1024) void seed_kernel(LadderArgs c, RowsArgs r, Ro
   __shared__ int16_t idx_l[CAPPED ? kMaxOrderRows : 1];
   const int lane_ix = blockIdx.x;
   const int b = lane_ix / c.n_groups, g = lane_ix % c.n_groups;
-  const int K = c.k_max, D = c.dk, J = (D + kWave - 1) / kWave;
+  const int K = c.k_max, D = c.dk;
   const int n = valid_rows(r, b);
   const int tid = static_cast<int>(threadIdx.x), nthr = static_cast<int>(blockDim.x);
   const int l = lane_id(), w = wave_id(), nw = nthr / kWave;
@@ -781,51 +849,63 @@ __global__ __launch_bounds__(1024) void seed_kernel(LadderArgs c, RowsArgs r, Ro
     n_use = 0;
   }
   if (n_use > 0 && tid == 0) picks_s[0] = pick;
-  // While seeding, the rows' running distances live in LDS (the candidate
-  // centers take the space afterwards); a wave takes kSeedRows rows at a time,
-  // their loads issued together, and holds the pick row in registers.
-  float* ds_l = cand_s;
-  constexpr int kSeedRows = 4, JM = kMaxDim / kWave;
+  // Rows as 16-byte units where the layout allows it.
+  const bool vec = (reinterpret_cast<uintptr_t>(r.k) & 15u) == 0 && r.k_sb % 8 == 0 && r.k_sg % 8 == 0 &&
+                   r.k_st % 8 == 0 && D % 8 == 0;
+  const int u = group_unit(), rr = l >> 3;
+  constexpr int kGroups = J <= 2 ? 2 : 1;   // 8-row groups of a wave whose loads are issued together
+  for (int s = tid; s < n; s += nthr) ord_l[s] = static_cast<uint16_t>(ord[s]);
+  __syncthreads();
+  auto load_row = [&](int s, uint4 (&x)[J]) {
+    load_units<J>(gp(kbase) + static_cast<int64_t>(ord_l[min(s, n - 1)]) * r.k_st, u, D, vec, x);
+  };
+  int steps = 0;
   for (int step = 0; step + 1 < n_use; ++step) {
     // dist = min(dist, d2(., pick)), with the pick itself masked; argmax -> next pick.
-    const uint16_t* prow = kbase + static_cast<int64_t>(ord[pick]) * r.k_st;
-    float xp[JM];
+    float xp[J][8];
+    {
+      uint4 x[J];
+      load_row(pick, x);
 #pragma unroll
-    for (int j = 0; j < JM; ++j) xp[j] = feat_or_zero(gp(prow), l + j * kWave, D);
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xp[j][i] = unit_feature<J>(x, j, i);
+    }
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
-    for (int s0 = w * kSeedRows; s0 < n; s0 += nw * kSeedRows) {
-      float x[kSeedRows][JM];
+    for (int s0 = w * 8 * kGroups; s0 < n; s0 += nw * 8 * kGroups) {
+      uint4 x[kGroups][J];
 #pragma unroll
-      for (int u = 0; u < kSeedRows; ++u) {
-        const uint16_t* row = kbase + static_cast<int64_t>(ord[min(s0 + u, n - 1)]) * r.k_st;
+      for (int q = 0; q < kGroups; ++q) load_row(s0 + 8 * q + rr, x[q]);
 #pragma unroll
-        for (int j = 0; j < JM; ++j) x[u][j] = feat_or_zero(gp(row), l + j * kWave, D);
-      }
-#pragma unroll
-      for (int u = 0; u < kSeedRows; ++u) {
-        const int s = s0 + u;
-        if (s >= n) break;
-        float e = 0.f;
-#pragma unroll
-        for (int j = 0; j < JM; ++j) {
-          if (j < J) {
-            const float diff = l + j * kWave < D ? x[u][j] - xp[j] : 0.f;
-            e = j == 0 ? diff * diff : e + diff * diff;
+      for (int q = 0; q < kGroups; ++q) {
+        const int s = s0 + 8 * q + rr;
+        const float d2 = group_d2<J>(x[q], xp, u);
+        if (s < n) {
+          float val, prev;
+          if (step == 0) {
+            prev = __builtin_inff();
+            val = as[s] < 0 ? d2 : -__builtin_inff();
+          } else {
+            prev = ds_l[s];
+            val = fminf(prev, d2);
+            if (prev != prev) prev = __builtin_inff();
           }
-        }
-        const float d2 = wave_sum0(e);
-        float val;
-        if (step == 0) val = as[s] < 0 ? d2 : -__builtin_inff();
-        else val = fminf(ds_l[s], d2);
-        if (s == pick) val = -__builtin_inff();
-        if (l == 0) ds_l[s] = val;
-        if (val > bv || (val == bv && s < bi)) {
-          bv = val;
-          bi = s;
+          if (s == pick) val = -__builtin_inff();
+          if ((l & 7) == 0) {
+            ds_l[s] = val;
+            if constexpr (!CAPPED) {
+              if (step == 0 || d2 < prev) arg_l[s] = static_cast<int8_t>(d2 < prev ? free_s[step] : 0);
+            }
+          }
+          if (val > bv || (val == bv && s < bi)) {
+            bv = val;
+            bi = s;
+          }
         }
       }
     }
+    ++steps;
     block_argmax(bv, bi, red_v, red_i);
     if (bi < 0 || bi >= n) {
       n_use = step + 1;
@@ -850,49 +930,49 @@ __global__ __launch_bounds__(1024) void seed_kernel(LadderArgs c, RowsArgs r, Ro
   for (int cc = 0; cc < K; ++cc) cand_bits |= (c.alive[lane_ix * K + cc] ? 1u : 0u) << cc;
   for (int k = 0; k < n_use; ++k) cand_bits |= 1u << free_s[k];
   if constexpr (!CAPPED) {
-    // Every orphan's nearest candidate, kSeedRows rows of a wave at a time.
-    for (int s0 = w * kSeedRows; s0 < n; s0 += nw * kSeedRows) {
-      float x[kSeedRows][JM];
-      bool orphan[kSeedRows];
+    // Every orphan's nearest candidate (the lowest cluster on ties): the nearest of the seeds
+    // passed so far, then the last seed and the live clusters.
+    const uint32_t seeds = [&] {
+      uint32_t m = 0;
+      for (int k = 0; k + 1 < n_use; ++k) m |= 1u << free_s[k];
+      return m;
+    }();
+    for (int s0 = w * 8 * kGroups; s0 < n; s0 += nw * 8 * kGroups) {
+      uint4 x[kGroups][J];
+      float best[kGroups];
+      int arg[kGroups];
 #pragma unroll
-      for (int u = 0; u < kSeedRows; ++u) {
-        orphan[u] = s0 + u < n && as[s0 + u] < 0;
-        const uint16_t* row = kbase + static_cast<int64_t>(ord[min(s0 + u, n - 1)]) * r.k_st;
-#pragma unroll
-        for (int j = 0; j < JM; ++j) x[u][j] = orphan[u] ? feat_or_zero(gp(row), l + j * kWave, D) : 0.f;
-      }
-      float best[kSeedRows];
-      int arg[kSeedRows];
-#pragma unroll
-      for (int u = 0; u < kSeedRows; ++u) {
-        best[u] = __builtin_inff();
-        arg[u] = 0;
+      for (int q = 0; q < kGroups; ++q) {
+        const int s = min(s0 + 8 * q + rr, n - 1);
+        load_row(s, x[q]);
+        best[q] = steps ? ds_l[s] : __builtin_inff();
+        if (best[q] != best[q]) best[q] = __builtin_inff();
+        arg[q] = steps ? arg_l[s] : 0;
       }
       for (int cc = 0; cc < K; ++cc) {
-        float cj[JM];
+        if (!(((cand_bits & ~seeds) >> cc) & 1u)) continue;
+        float cj[J][8];
 #pragma unroll
-        for (int j = 0; j < JM; ++j) cj[j] = j < J && l + j * kWave < D ? cand_s[cc * D + l + j * kWave] : 0.f;
-        const bool cand = (cand_bits >> cc) & 1u;
+        for (int j = 0; j < J; ++j)
 #pragma unroll
-        for (int u = 0; u < kSeedRows; ++u) {
-          float e = 0.f;
-#pragma unroll
-          for (int j = 0; j < JM; ++j) {
-            if (j < J) {
-              const float diff = l + j * kWave < D ? x[u][j] - cj[j] : 0.f;
-              e = j == 0 ? diff * diff : e + diff * diff;
-            }
+          for (int i = 0; i < 8; ++i) {
+            const int d = 64 * j + 8 * u + i;
+            cj[j][i] = d < D ? cand_s[cc * D + d] : 0.f;
           }
-          e = wave_sum0(e);
-          if (cand && e < best[u]) {
-            best[u] = e;
-            arg[u] = cc;
+#pragma unroll
+        for (int q = 0; q < kGroups; ++q) {
+          const float e = group_d2<J>(x[q], cj, u);
+          if (e < best[q] || (e == best[q] && cc < arg[q])) {
+            best[q] = e;
+            arg[q] = cc;
           }
         }
       }
 #pragma unroll
-      for (int u = 0; u < kSeedRows; ++u)
-        if (orphan[u] && l == 0) as[s0 + u] = static_cast<int8_t>(arg[u]);
+      for (int q = 0; q < kGroups; ++q) {
+        const int s = s0 + 8 * q + rr;
+        if (s < n && (l & 7) == 0 && as[s] < 0) as[s] = static_cast<int8_t>(arg[q]);
+      }
     }
     __syncthreads();
     if (tid < n_use) as[picks_s[tid]] = static_cast<int8_t>(free_s[tid]);
@@ -916,22 +996,20 @@ __global__ __launch_bounds__(1024) void seed_kernel(LadderArgs c, RowsArgs r, Ro
     float* cd = cap_dist + static_cast<int64_t>(lane_ix) * r.tokens * K;
     for (int i = w; i < n_rest; i += nw) {
       const int s = idx_l[i];
-      float x[kMaxDim / kWave];
+      float x[J];
       const uint16_t* row = kbase + static_cast<int64_t>(ord[s]) * r.k_st;
 #pragma unroll
-      for (int j = 0; j < kMaxDim / kWave; ++j) {
+      for (int j = 0; j < J; ++j) {
         const int d = l + j * kWave;
         x[j] = feat_or_zero(gp(row), d, D);
       }
       for (int cc = 0; cc < K; ++cc) {
         float e = 0.f;
 #pragma unroll
-        for (int j = 0; j < kMaxDim / kWave; ++j) {
-          if (j < J) {
-            const int d = l + j * kWave;
-            const float diff = d < D ? x[j] - cand_s[cc * D + d] : 0.f;
-            e = j == 0 ? diff * diff : e + diff * diff;
-          }
+        for (int j = 0; j < J; ++j) {
+          const int d = l + j * kWave;
+          const float diff = d < D ? x[j] - cand_s[cc * D + d] : 0.f;
+          e = j == 0 ? diff * diff : e + diff * diff;
         }
         e = wave_sum0(e);
         if (l == 0) cd[static_cast<int64_t>(i) * K + cc] = ((cand_bits >> cc) & 1u) ? e : __builtin_inff();
@@ -1010,12 +1088,19 @@ int launch_route(const LadderArgs& c, const RowsArgs& r, const RouteParams& p, c
     else if (nj == 3) ok = attach(attach_kernel<3>, attach_tile<3>(), attach_shmem<3>(c.k_max));
     else ok = attach(attach_kernel<4>, attach_tile<4>(), attach_shmem<4>(c.k_max));
     if (!ok) return LOGKV_ERUNTIME;
-    if (p.hard_cap > 0.f)
-      hipLaunchKernelGGL(seed_kernel<true>, dim3(lanes), dim3(1024), 0, stream, c, r, p, ws.order, ws.assign,
-                         ws.s_win, ws.dist, ws.cap_dist);
-    else
-      hipLaunchKernelGGL(seed_kernel<false>, dim3(lanes), dim3(1024), 0, stream, c, r, p, ws.order, ws.assign,
-                         ws.s_win, ws.dist, static_cast<float*>(nullptr));
+    auto seed = [&](auto capped, auto slices) {
+      constexpr bool kCapped = decltype(capped)::value;
+      hipLaunchKernelGGL((seed_kernel<kCapped, decltype(slices)::value>), dim3(lanes), dim3(1024), 0, stream, c, r, p,
+                         ws.order, ws.assign, ws.s_win, kCapped ? ws.cap_dist : static_cast<float*>(nullptr));
+    };
+    auto by_slices = [&](auto capped) {
+      if (nj == 1) seed(capped, std::integral_constant<int, 1>{});
+      else if (nj == 2) seed(capped, std::integral_constant<int, 2>{});
+      else if (nj == 3) seed(capped, std::integral_constant<int, 3>{});
+      else seed(capped, std::integral_constant<int, 4>{});
+    };
+    if (p.hard_cap > 0.f) by_slices(std::true_type{});
+    else by_slices(std::false_type{});
   }
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }

@@ -44,7 +44,6 @@ struct Workspace {
   int32_t* order;      // [n_batch, T]
   int8_t* assign;      // [lanes, T]
   float* s_win;        // [lanes, T]
-  float* dist;         // [lanes, T]
   float* cap_dist;     // [lanes, T, K] orphan-to-candidate distances of a capped route (shares the
                        // ladder scratch, which only the commit launches after the route use)
   uint8_t* snap_alive; // [lanes, K] alive flags before the commit (written by its ladder blocks)
