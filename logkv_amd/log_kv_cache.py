@@ -98,6 +98,37 @@ class _SemanticReplayUpdates:
         return len(self.tensors) - 1
 
 
+class _HostOpLog:
+    """A finished op-log's rows on the host: ``rows`` int32 ``[Bt, G, max_len, 4]`` and ``lengths``
+    ``[Bt, G]``, both copies. Row tuples are built where they are read (``lists()``, indexing): a
+    training step over 4096 tokens keeps 30K rows that only a failed check would ever print."""
+
+    __slots__ = ("_rows", "_lengths", "_frozen")
+
+    def __init__(self, rows, lengths):
+        self._rows, self._lengths, self._frozen = rows, lengths, None
+
+    def lists(self):
+        """Fresh ``[Bt][G]`` lists of (op, cluster, arg, position) tuples."""
+        lens = self._lengths.tolist()
+        return [[list(map(tuple, lane[:n].tolist())) for lane, n in zip(batch, row)]
+                for batch, row in zip(self._rows, lens)]
+
+    def _tuples(self):
+        if self._frozen is None:
+            self._frozen = tuple(tuple(map(tuple, batch)) for batch in self.lists())
+        return self._frozen
+
+    def __len__(self):
+        return self._rows.size(0)
+
+    def __getitem__(self, i):
+        return self._tuples()[i]
+
+    def __iter__(self):
+        return iter(self._tuples())
+
+
 class _SemanticReplayPlans:
     """Host-only replay state of one invocation (litgpt/log_kv_cache.py:97-108).
 
@@ -110,7 +141,8 @@ class _SemanticReplayPlans:
     def __init__(self, host_log):
         if host_log is None:
             raise RuntimeError("semantic replay plans require an existing CPU op-log")
-        self.host_log = tuple(tuple(tuple(map(tuple, lane)) for lane in batch) for batch in host_log)
+        self.host_log = (host_log if isinstance(host_log, _HostOpLog) else
+                         tuple(tuple(tuple(map(tuple, lane)) for lane in batch) for batch in host_log))
         self.plans = {}
 
 
@@ -387,7 +419,7 @@ class LogStructuredKVCache(nn.Module):
         self.op_log: torch.Tensor | None = None
         self.op_log_len: torch.Tensor | None = None
         self._op_replay_cursor_host = None
-        self._last_op_log_host = None
+        self._op_log_host = self._op_log_lists = None
         # Update tape (semantic_replay_updates): the bound tape, whether it is
         # replayed, and the flushes recorded / replayed since the log began.
         self._active_updates = None
@@ -741,8 +773,8 @@ class LogStructuredKVCache(nn.Module):
     def take_op_log(self):
         """(log ``[Bt, G, max_len, 4]``, lengths ``[Bt, G]``) copies (litgpt/log_kv_cache.py:2029-2038).
 
-        Reads the lengths back (one synchronisation) and keeps the rows as host
-        tuples in ``_last_op_log_host``. Raises ``RuntimeError`` when a lane
+        Reads the lengths and the rows back; ``_last_op_log_host`` gives the rows
+        as host tuples. Raises ``RuntimeError`` when a lane
         logged more rows than the capacity (the rows past it were not written).
         """
         if getattr(self, "op_log", None) is None or getattr(self, "op_log_len", None) is None:
@@ -752,11 +784,16 @@ class LogStructuredKVCache(nn.Module):
         if int(lengths.max()) > self.op_log.size(2):
             raise RuntimeError("semantic LogKV op_log overflow")
         max_len = int(lengths.max())
-        rows = self.op_log[:, :, :max_len].cpu().tolist()
-        lens = lengths.tolist()
-        self._last_op_log_host = [[[tuple(r) for r in rows[b][g][:lens[b][g]]] for g in range(self.n_groups)]
-                                  for b in range(self.batch_size)]
+        self._op_log_host = _HostOpLog(self.op_log[:, :, :max_len].cpu(), lengths)
+        self._op_log_lists = None
         return self.op_log[:, :, :max_len].clone(), self.op_log_len.clone()
+
+    @property
+    def _last_op_log_host(self):
+        """``[Bt][G]`` lists of the last taken log's row tuples (None before any); built on first read."""
+        if self._op_log_host is not None and self._op_log_lists is None:
+            self._op_log_lists = self._op_log_host.lists()
+        return self._op_log_lists
 
     def _replay_flush(self, k_raw, v, positions, positions_host, counts, log, lengths, log_host, plans):
         """Re-apply one logged flush (litgpt/log_kv_cache.py:5067-5114) on the device.
@@ -1279,7 +1316,7 @@ class LogKVStreamTrainingAttention(torch.autograd.Function):
                                      record_op_log=True, span_ends=None if ctx.span_ends is None else
                                      [row[start:end] for row in ctx.span_ends])
         op_log, op_log_len = cache.take_op_log()
-        ctx.replay_plans = _SemanticReplayPlans(cache._last_op_log_host)
+        ctx.replay_plans = _SemanticReplayPlans(cache._op_log_host)
         ctx.op_log, ctx.op_log_len, ctx.op_log_host = op_log, op_log_len, ctx.replay_plans.host_log
         ctx.updates, ctx.plans, ctx.cache = updates, plans, cache
         ctx.scale, ctx.train_block, ctx.second_order_scale = scale, train_block, second_order_scale
