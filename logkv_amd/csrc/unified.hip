@@ -838,10 +838,17 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_plan_kernel(ReduceArgs 
 // that is not kept, its mirror; the screen leaves only the elements that can
 // hold the kept row's minimum key (an atomic minimum per tile) or lower a
 // column's cached minimum to evaluate ward_cost.
-constexpr int kLwCols = 4, kLwRows = 16, kLwTile = kLwCols * kWave;
+// The mirrors were three quarters of the phase: written as the rows were
+// computed, a store met 64 different matrix rows. The tile's values go through
+// LDS instead and a store writes 4 rows x the tile's 16 kept columns, which
+// share cache lines. First round of a 4096-row flush, 32 lanes: 1.21 -> 0.91 ms.
+constexpr int kLwCols = 2, kLwRows = 16, kLwTile = kLwCols * kWave;
+constexpr int kLwLd = kLwTile + 4;   // LDS row stride: a store's 16 rows x 4 columns fall into distinct banks
 
 template <bool LIMIT>
 __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) {
+  __shared__ float tile_s[kPhaseWaves][kLwRows * kLwLd];
+  __shared__ int mirror_s[kPhaseWaves][kLwTile];   // a column's matrix row, -1 where it takes no mirror
   const int lane = blockIdx.y, M = a.M, l = lane_id();
   const LaneCtl ctl = a.ctl[lane];
   if (!ctl.work) return;
@@ -855,11 +862,13 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
   // Merges per item: up to kLwRows, fewer when that would leave waves idle.
   const int rows = max(1, min(kLwRows, n_ok * col_chunks / waves));
   const int items = col_chunks * ((n_ok + rows - 1) / rows);
+  float* tile = tile_s[wave_id()];
+  int* mirror = mirror_s[wave_id()];
   for (int it = blockIdx.x * kPhaseWaves + wave_id(); it < items; it += waves) {
     const int pg = it / col_chunks, cc = it - pg * col_chunks;
-    int col[kLwCols];
+    int col[kLwCols], mate[kLwCols];
     uint8_t fl[kLwCols];
-    float mc[kLwCols], rc[kLwCols], thr[kLwCols];
+    float mc[kLwCols], rc[kLwCols], thr[kLwCols], qa[kLwCols], qb[kLwCols], qs[kLwCols];
 #pragma unroll
     for (int e = 0; e < kLwCols; ++e) {
       const int idx = cc * kLwTile + e * kWave + l;
@@ -871,43 +880,75 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
       // A kept or rescanned column takes no push (-1); keys only fall during
       // the phase, so the cost read now bounds every key that can still lower it.
       thr[e] = col[e] >= 0 && !(fl[e] & (kKeep | kDirty)) ? key_cost(s.packed[c]) : -1.f;
+      // A kept column's own merge.
+      mate[e] = 0;
+      qa[e] = qb[e] = qs[e] = 0.f;
+      if (fl[e] & kKeep) {
+        const int pc = s.pair_of[c];
+        mate[e] = s.best[c];
+        qa[e] = s.p_alpha[pc], qb[e] = s.p_beta[pc], qs[e] = s.p_shift[pc];
+      }
+      mirror[e * kWave + l] = fl[e] & kKeep ? -1 : col[e];
     }
-    const int p1 = min(n_ok, (pg + 1) * rows);
-    for (int j = pg * rows; j < p1; ++j) {
-      const int ra = kept[j], rb = s.best[ra], p = s.pair_of[ra];
-      const float alpha = s.p_alpha[p], beta = s.p_beta[p], shift = s.p_shift[p];
-      const float total = s.mass[ra], rad = s.radius[ra];
-      float* row_a = dist + static_cast<int64_t>(ra) * M;
+    // The item's merges, one per lane, read back by lane number; a row's
+    // elements are loaded while the row before it is computed (no write of the
+    // phase reaches an element that it reads: kept rows' live columns are
+    // written by their own wave only, retired rows and columns by none).
+    const int j0 = pg * rows, nj = min(n_ok, j0 + rows) - j0;
+    const int my_a = kept[j0 + min(l, nj - 1)], my_b = s.best[my_a], my_p = s.pair_of[my_a];
+    const float my_alpha = s.p_alpha[my_p], my_beta = s.p_beta[my_p], my_shift = s.p_shift[my_p];
+    const float my_total = s.mass[my_a], my_rad = s.radius[my_a];
+    float x_aa[kLwCols], x_ba[kLwCols], x_ab[kLwCols], x_bb[kLwCols];
+    auto load = [&](int j) {
+      const int ra = __builtin_amdgcn_readlane(my_a, j), rb = __builtin_amdgcn_readlane(my_b, j);
+      const float* row_a = dist + static_cast<int64_t>(ra) * M;
       const float* row_b = dist + static_cast<int64_t>(rb) * M;
-      float x_aa[kLwCols], x_ba[kLwCols], nw[kLwCols], sc[kLwCols];
-      bool border[kLwCols];
 #pragma unroll
       for (int e = 0; e < kLwCols; ++e) {
         const int c = col[e] >= 0 ? col[e] : ra;
         x_aa[e] = row_a[c];
         x_ba[e] = row_b[c];
+        if (fl[e] & kKeep) {
+          x_ab[e] = row_a[mate[e]];
+          x_bb[e] = row_b[mate[e]];
+        }
       }
-      float m = __builtin_inff();
+    };
+    auto lane_f32 = [](float x, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), j)); };
+#pragma unroll
+    for (int e = 0; e < kLwCols; ++e) x_ab[e] = x_bb[e] = 0.f;
+    load(0);
+    for (int j = 0; j < nj; ++j) {
+      const int ra = __builtin_amdgcn_readlane(my_a, j);
+      const float alpha = lane_f32(my_alpha, j), beta = lane_f32(my_beta, j), shift = lane_f32(my_shift, j);
+      const float total = lane_f32(my_total, j), rad = lane_f32(my_rad, j);
+      float* row_a = dist + static_cast<int64_t>(ra) * M;
+      float nw[kLwCols], sc[kLwCols];
+      bool border[kLwCols];
 #pragma unroll
       for (int e = 0; e < kLwCols; ++e) {
         const int c = col[e];
         float v = alpha * x_aa[e] + beta * x_ba[e] - shift;
         if (c >= 0 && (fl[e] & kKeep) && c != ra) {
-          const int q = s.best[c], pc = s.pair_of[c];
-          const float qa = s.p_alpha[pc], qb = s.p_beta[pc], qs = s.p_shift[pc];
-          const float x_ab = row_a[q], x_bb = row_b[q];
-          const float own = qa * v + qb * (alpha * x_ab + beta * x_bb - shift) - qs;
-          const float other = alpha * (qa * x_aa[e] + qb * x_ab - qs) + beta * (qa * x_ba[e] + qb * x_bb - qs) - shift;
+          const float own = qa[e] * v + qb[e] * (alpha * x_ab[e] + beta * x_bb[e] - shift) - qs[e];
+          const float other = alpha * (qa[e] * x_aa[e] + qb[e] * x_ab[e] - qs[e]) +
+                              beta * (qa[e] * x_ba[e] + qb[e] * x_bb[e] - qs[e]) - shift;
           v = ra < c ? own : other;
         }
         v = v < 0.f ? 0.f : v;
         if (c == ra) v = 0.f;
         nw[e] = v;
+      }
+      if (j + 1 < nj) load(j + 1);
+      float m = __builtin_inff();
+#pragma unroll
+      for (int e = 0; e < kLwCols; ++e) {
+        const int c = col[e];
         if (c >= 0) {
-          row_a[c] = v;
-          if (!(fl[e] & kKeep)) dist[static_cast<int64_t>(c) * M + ra] = v;
+          row_a[c] = nw[e];
         }
-        sc[e] = screen_cost<LIMIT>(v, total, mc[e], rad, rc[e], limit, c >= 0 && c != ra, border[e]);
+        tile[j * kLwLd + e * kWave + l] = nw[e];
+        sc[e] = screen_cost<LIMIT>(nw[e], total, mc[e], rad, rc[e], limit, c >= 0 && c != ra, border[e]);
         if (!border[e]) m = sc[e] < m ? sc[e] : m;
       }
       const float cut = screen_cutoff(__uint_as_float(wave_min_u32(__float_as_uint(m))));
@@ -929,6 +970,17 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
       if (l == 0 && best < kInfKey)
         atomicMin(reinterpret_cast<unsigned long long*>(&s.packed[ra]), static_cast<unsigned long long>(best));
     }
+    // The mirrors: lane l writes kept column l % 16 of tile column 4 i + l / 16. The wave's own LDS
+    // (its accesses complete in order; the fences keep the compiler's order).
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int jj = l & (kLwRows - 1), ra = __shfl(my_a, jj, kWave);
+    for (int i = 0; i < kLwTile / 4; ++i) {
+      const int e = 4 * i + l / kLwRows, c = mirror[e];
+      if (c >= 0 && jj < nj) dist[static_cast<int64_t>(c) * M + ra] = tile[jj * kLwLd + e];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -966,15 +1018,27 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_rescan_kernel(ReduceArgs
       mc[e] = col[e] >= 0 ? s.mass[col[e]] : 0.f;
       rc[e] = col[e] >= 0 ? s.radius[col[e]] : 0.f;
     }
-    const int q1 = min(n_dirty, (rg + 1) * rows);
-    for (int q = rg * rows; q < q1; ++q) {
-      const int r = dirty[q];
-      const float mr = s.mass[r], rr = s.radius[r];
-      const float* row = dist + static_cast<int64_t>(r) * M;
+    // The item's rows, one per lane, read back by lane number; the next row's
+    // elements are loaded while a row is screened.
+    const int q0 = rg * rows, nq = min(n_dirty, q0 + rows) - q0;
+    const int my_r = dirty[q0 + min(l, nq - 1)];
+    const float my_mass = s.mass[my_r], my_rad = s.radius[my_r];
+    float next[kScanCols];
+    auto load = [&](int q) {
+      const float* row = dist + static_cast<int64_t>(__builtin_amdgcn_readlane(my_r, q)) * M;
+#pragma unroll
+      for (int e = 0; e < kScanCols; ++e) next[e] = row[col[e] >= 0 ? col[e] : 0];
+    };
+    load(0);
+    for (int q = 0; q < nq; ++q) {
+      const int r = __builtin_amdgcn_readlane(my_r, q);
+      const float mr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_mass), q));
+      const float rr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_rad), q));
       float d2[kScanCols], sc[kScanCols];
       bool border[kScanCols];
 #pragma unroll
-      for (int e = 0; e < kScanCols; ++e) d2[e] = row[col[e] >= 0 ? col[e] : 0];
+      for (int e = 0; e < kScanCols; ++e) d2[e] = next[e];
+      if (q + 1 < nq) load(q + 1);
       float m = __builtin_inff();
 #pragma unroll
       for (int e = 0; e < kScanCols; ++e) {
