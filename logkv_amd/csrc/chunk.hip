@@ -7,7 +7,7 @@
 // v_mfma_f32_32x32x16_bf16: a block of 8 waves (one per CU, two per SIMD)
 // owns 256 query rows of one KV group, a wave 32 of them (one per lane
 // column), so each staged K / V tile serves 256 queries. Per 64-row key tile,
-// staged in LDS (K row-major, V transposed):
+// staged row-major in LDS (V read transposed):
 //   S^T = K Q^T   (keys x queries; each lane holds 16 keys of its own query),
 //   online softmax per lane (its query's max and sum, the other 16 keys of the
 //   32-key block in lane ^ 32),
@@ -22,6 +22,11 @@
 //   binades, or holds an infinity, NaN or subnormal, reads its bf16 V rows
 //   instead and splits P 2^15 into high and low bf16 parts (two products per
 //   step, P kept to about 2^-16).
+// V is staged row-major and read transposed by ds_read_b64_tr_b16: 2048 rows of
+// 16 heads over 19K packed rows 248 us, with the transpose done by byte
+// permutes and 4-byte LDS stores while staging 268 us. Matrix cores are busy a
+// third of the cycles and the vector unit (the exponentials) two fifths, one
+// after the other: the two waves of a SIMD run in step.
 // Queries live in registers for the whole key range; the K / V tiles are
 // double-buffered in LDS with one barrier per tile.
 // The P^T operand is the lane's own score registers: MFMA B operand element j
@@ -43,6 +48,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWavesPerBlock = 8;                 // waves per block, each owning 32 query rows
 constexpr int kThreads = 64 * kWavesPerBlock;
@@ -51,15 +57,13 @@ constexpr int kBlocksPerCu = 8 / kWavesPerBlock;  // resident blocks per CU (two
 constexpr int kKeys = 64;        // key rows per staged tile
 constexpr int kMaxSteps = 9;     // 16-wide steps of the packed width (<= 144)
 constexpr int kLdK = 152;        // K tile row stride in LDS (bf16)
-constexpr int kLdV = kKeys + 4;  // V^T row stride in LDS (bf16; 34 dwords: 16 rows' 8-byte reads hit distinct banks)
+constexpr int kLdV = 144;        // V tile row stride in LDS (72 dwords: the 4 rows of a transposed read hit distinct banks)
 constexpr int kMaxDvBlocks = 4;  // dv <= 128
 constexpr int kVSlices = 64;     // row slices of a lane's V in the fp16 copy
 // vshift of a lane whose V has no exact fp16 copy (the bf16 path reads its rows).
 constexpr int kBf16Lane = 1 << 20;
 // P is scaled by 2^kPShift before its fp16 rounding (P <= 1, so P 2^15 < 65504).
 constexpr int kPShift = 15;
-
-__device__ __forceinline__ __bf16 to_bf16(float x) { return static_cast<__bf16>(x); }
 
 // max / sum of the values of lanes l and l ^ 32, in every lane: one permlane
 // swap leaves {x[l], x[l ^ 32]} in its two results (lower-half lane's value
@@ -71,6 +75,18 @@ __device__ __forceinline__ float pair_max32(float x) {
 __device__ __forceinline__ float pair_sum32(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// V^T operand of a row-major V tile: for feature f0 + lane % 32, keys 16 st + 8 (j / 4) + 4 (lane / 32)
+// + j % 4, the order of the score registers (ds_read_b64_tr_b16 turns a 16-lane group's 4 rows x 16
+// features, lane i reading row i / 4, features 4 (i % 4) .. + 4, into 4 rows of feature i per lane).
+__device__ __forceinline__ uint4 load_vt(const uint16_t* tile, int f0, int st) {
+  typedef __attribute__((address_space(3))) s16x4* lds4;
+  const int l = lane_id(), i = l & 15, h = l >> 5;
+  const uint16_t* p = tile + (16 * st + 4 * h + (i >> 2)) * kLdV + f0 + (l & 16) + 4 * (i & 3);
+  const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p)));
+  const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(p + 8 * kLdV)));
+  return make_uint4(x.x, x.y, y.x, y.y);
 }
 
 // The block's logical (query block, split, lane) in a grid of (query blocks,
@@ -98,17 +114,17 @@ __device__ __forceinline__ ChunkBlock chunk_block() {
 // and writes partials [m, l, acc[dv]] per query (m in the base-2 domain).
 // NKS 16-wide steps of the packed width and NDV 32-wide blocks of dv at
 // compile time (straight-line tile code); columns past the packed width and
-// V^T rows past dv are zero, so a kernel with more steps or blocks than the
+// V columns past dv are zero, so a kernel with more steps or blocks than the
 // shape needs gives the same result.
 // BF16V: the body of a lane without an exact fp16 V copy (vshift kBf16Lane).
 template <int NKS, int NDV, bool BF16V>
 __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const int32_t* __restrict__ width_ptr,
                                            int splits, float* __restrict__ part, const uint16_t* __restrict__ v16,
                                            int kv, const ChunkBlock blk_id) {
-  // Two K / V^T tile buffers: tile i + 1 is written into the other buffer while
+  // Two K / V tile buffers: tile i + 1 is written into the other buffer while
   // tile i is read, so one barrier per tile orders both.
   __shared__ __align__(16) uint16_t k_s[2][kKeys * kLdK];
-  __shared__ __align__(16) uint16_t vt_s[2][kMaxDvBlocks * 32 * kLdV];
+  __shared__ __align__(16) uint16_t v_s[2][kKeys * kLdV];
   const int lane_ix = blk_id.lane, split = blk_id.split, G = a.n_groups;
   const int b = lane_ix / G, g = lane_ix % G;
   const int rep = a.n_heads / G, nq = rep * a.tq;
@@ -145,16 +161,11 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
                                                      e[4] | (uint32_t(e[5]) << 16), e[6] | (uint32_t(e[7]) << 16)));
     }
   }
-  // Columns past the packed width and V^T rows past dv stay zero in every
-  // tile of both buffers.
+  // Columns past the packed width stay zero in every tile of both buffers.
   for (int i = threadIdx.x; i < 2 * kKeys * (kLdK - dim); i += blockDim.x) {
     const int bf = i / (kKeys * (kLdK - dim)), rest = i - bf * kKeys * (kLdK - dim);
     const int r = rest / (kLdK - dim), c = dim + rest % (kLdK - dim);
     k_s[bf][r * kLdK + c] = 0;
-  }
-  for (int i = threadIdx.x; i < 2 * (32 * NDV - a.dv) * kLdV; i += blockDim.x) {
-    const int bf = i / ((32 * NDV - a.dv) * kLdV), rest = i - bf * (32 * NDV - a.dv) * kLdV;
-    vt_s[bf][a.dv * kLdV + rest] = 0;
   }
   f32x16 o[NDV];
 #pragma unroll
@@ -168,10 +179,10 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
                                         : gp(v16) + static_cast<int64_t>(lane_ix) * a.cap * a.dv;
   const int vstride = BF16V ? dim : a.dv;
   const int units = dim / 8;
-  const int vunits = a.dv / 8;
   // Each thread's staging tasks are the same in every tile: up to kKTasks
-  // 16-byte K units (row, unit) and kVTasks V tasks (key pair, 8-wide dv unit).
-  constexpr int kKTasks = (kKeys * kMaxSteps * 2 + kThreads - 1) / kThreads, kVTasks = (kKeys / 2) * 16 / kThreads;
+  // 16-byte K units and kVTasks V units (row, unit; zero past dv).
+  constexpr int kUnitsV = 4 * NDV;
+  constexpr int kKTasks = (kKeys * kMaxSteps * 2 + kThreads - 1) / kThreads, kVTasks = kKeys * kUnitsV / kThreads;
   int k_row[kKTasks], k_goff[kKTasks], k_loff[kKTasks];
 #pragma unroll
   for (int q = 0; q < kKTasks; ++q) {
@@ -182,15 +193,8 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
     k_goff[q] = 8 * u;
     k_loff[q] = r * kLdK + 8 * u;
   }
-  int v_pair[kVTasks], v_unit[kVTasks];
-#pragma unroll
-  for (int q = 0; q < kVTasks; ++q) {
-    const int i = threadIdx.x + kThreads * q;
-    v_pair[q] = i < (kKeys / 2) * vunits ? i % (kKeys / 2) : -1;
-    v_unit[q] = i / (kKeys / 2);
-  }
   // Registers of the next tile (loaded while the current one is computed).
-  uint4 kx[kKTasks], vx[kVTasks][2];
+  uint4 kx[kKTasks], vx[kVTasks];
   auto load_tile = [&](int t0) {
     const int rows = min(kKeys, k_stop - t0);
 #pragma unroll
@@ -201,33 +205,21 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
     }
 #pragma unroll
     for (int q = 0; q < kVTasks; ++q) {
-      const int kp = v_pair[q] < 0 ? 0 : v_pair[q];
-      const int r0 = min(2 * kp, rows - 1), r1 = min(2 * kp + 1, rows - 1);
-      vx[q][0] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + r0) * vstride + 8 * v_unit[q]);
-      vx[q][1] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + r1) * vstride + 8 * v_unit[q]);
-      if (2 * kp >= rows) vx[q][0] = make_uint4(0, 0, 0, 0);
-      if (2 * kp + 1 >= rows) vx[q][1] = make_uint4(0, 0, 0, 0);
+      const int i = threadIdx.x + kThreads * q, r = i / kUnitsV, u = i % kUnitsV;
+      const bool on = r < rows && 8 * u < a.dv;
+      vx[q] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + (on ? r : 0)) * vstride + (on ? 8 * u : 0));
+      if (!on) vx[q] = make_uint4(0, 0, 0, 0);
     }
   };
-  // K rows row-major; V transposed: each task's two key rows of one 8-wide dv
-  // unit become 8 dwords (key pairs). Rows past the end are zeros.
+  // Both row-major; rows past the end are zeros.
   auto store_tile = [&](int bf) {
 #pragma unroll
     for (int q = 0; q < kKTasks; ++q)
       if (k_row[q] < kKeys) *reinterpret_cast<uint4*>(&k_s[bf][k_loff[q]]) = kx[q];
 #pragma unroll
     for (int q = 0; q < kVTasks; ++q) {
-      if (v_pair[q] < 0) continue;
-      const uint32_t a0[4] = {vx[q][0].x, vx[q][0].y, vx[q][0].z, vx[q][0].w};
-      const uint32_t a1[4] = {vx[q][1].x, vx[q][1].y, vx[q][1].z, vx[q][1].w};
-      const int r0 = 2 * v_pair[q], u = v_unit[q];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t lo = __builtin_amdgcn_perm(a1[j], a0[j], 0x05040100u);   // low halves of rows r0, r0 + 1
-        const uint32_t hi = __builtin_amdgcn_perm(a1[j], a0[j], 0x07060302u);   // high halves
-        *reinterpret_cast<uint32_t*>(&vt_s[bf][(8 * u + 2 * j) * kLdV + r0]) = lo;
-        *reinterpret_cast<uint32_t*>(&vt_s[bf][(8 * u + 2 * j + 1) * kLdV + r0]) = hi;
-      }
+      const int i = threadIdx.x + kThreads * q;
+      *reinterpret_cast<uint4*>(&v_s[bf][(i / kUnitsV) * kLdV + 8 * (i % kUnitsV)]) = vx[q];
     }
   };
   const int ntiles = k_begin < k_stop ? (k_stop - k_begin + kKeys - 1) / kKeys : 0;
@@ -246,7 +238,7 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
     const int t0 = k_begin + it * kKeys, bf = it & 1;
     const int rows = min(kKeys, k_stop - t0);
     const uint16_t* kt = k_s[bf];
-    const uint16_t* vt = vt_s[bf];
+    const uint16_t* vt = v_s[bf];
     // S^T = K Q^T over the packed width, the two 32-key blocks' chains
     // interleaved.
     f32x16 s[2];
@@ -328,10 +320,7 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
         const bf16x8 pl = __builtin_bit_cast(bf16x8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
 #pragma unroll
         for (int blk = 0; blk < NDV; ++blk) {
-          const uint16_t* vr = vt + (32 * blk + col) * kLdV + 16 * st + 4 * h;
-          const uint2 v0 = *reinterpret_cast<const uint2*>(vr);
-          const uint2 v1 = *reinterpret_cast<const uint2*>(vr + 8);
-          const bf16x8 vb = __builtin_bit_cast(bf16x8, make_uint4(v0.x, v0.y, v1.x, v1.y));
+          const bf16x8 vb = __builtin_bit_cast(bf16x8, load_vt(vt, 32 * blk, st));
           o[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vb, ph, o[blk], 0, 0, 0);
           o[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vb, pl, o[blk], 0, 0, 0);
         }
@@ -351,12 +340,7 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
                                                             __builtin_bit_cast(uint32_t, pw[3])));
       f16x8 vf[NDV];
 #pragma unroll
-      for (int blk = 0; blk < NDV; ++blk) {
-        const uint16_t* vr = vt + (32 * blk + col) * kLdV + 16 * st + 4 * h;
-        const uint2 v0 = *reinterpret_cast<const uint2*>(vr);
-        const uint2 v1 = *reinterpret_cast<const uint2*>(vr + 8);
-        vf[blk] = __builtin_bit_cast(f16x8, make_uint4(v0.x, v0.y, v1.x, v1.y));
-      }
+      for (int blk = 0; blk < NDV; ++blk) vf[blk] = __builtin_bit_cast(f16x8, load_vt(vt, 32 * blk, st));
 #pragma unroll
       for (int blk = 0; blk < NDV; ++blk) o[blk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[blk], ph, o[blk], 0, 0, 0);
     }
