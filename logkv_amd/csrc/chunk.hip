@@ -59,6 +59,8 @@ constexpr int kMaxSteps = 9;     // 16-wide steps of the packed width (<= 144)
 constexpr int kLdK = 152;        // K tile row stride in LDS (bf16)
 constexpr int kLdV = 144;        // V tile row stride in LDS (72 dwords: the 4 rows of a transposed read hit distinct banks)
 constexpr int kMaxDvBlocks = 4;  // dv <= 128
+constexpr int kMaxChunkSplits = 16;
+constexpr int kPartTail = 4;     // a partial's maximum and sum, padded to 16 bytes
 constexpr int kVSlices = 64;     // row slices of a lane's V in the fp16 copy
 // vshift of a lane whose V has no exact fp16 copy (the bf16 path reads its rows).
 constexpr int kBf16Lane = 1 << 20;
@@ -111,7 +113,7 @@ __device__ __forceinline__ ChunkBlock chunk_block() {
 
 // splits == 1: the block writes the output. splits > 1: block (x, s) covers the
 // s-th of `splits` equal parts (whole 64-row tiles) of its queries' key range
-// and writes partials [m, l, acc[dv]] per query (m in the base-2 domain).
+// and writes partials [acc[dv], m, l, 0, 0] per query (m in the base-2 domain).
 // NKS 16-wide steps of the packed width and NDV 32-wide blocks of dv at
 // compile time (straight-line tile code); columns past the packed width and
 // V columns past dv are zero, so a kernel with more steps or blocks than the
@@ -358,20 +360,15 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
   for (int it = n_full; it < ntiles; ++it) tile(it, std::true_type{});
   if (!q_ok) return;
   if (splits > 1) {
-    float* pp = part + ((static_cast<int64_t>(lane_ix) * splits + split) * nq + qi) * (a.dv + 2);
-    if (h == 0) {
-      pp[0] = m;
-      pp[1] = lsum;
-    }
+    float* pp = part + ((static_cast<int64_t>(lane_ix) * splits + split) * nq + qi) * (a.dv + kPartTail);
+    if (h == 0) *reinterpret_cast<float2*>(pp + a.dv) = make_float2(m, lsum);
 #pragma unroll
     for (int blk = 0; blk < NDV; ++blk) {
       if (blk < ndv) {
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          const int d = 32 * blk + 8 * i4 + 4 * h;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) pp[2 + d + j] = o[blk][4 * i4 + j];
-        }
+        for (int i4 = 0; i4 < 4; ++i4)
+          *reinterpret_cast<float4*>(pp + 32 * blk + 8 * i4 + 4 * h) =
+              make_float4(o[blk][4 * i4], o[blk][4 * i4 + 1], o[blk][4 * i4 + 2], o[blk][4 * i4 + 3]);
       }
     }
     return;
@@ -506,7 +503,9 @@ __global__ __launch_bounds__(256) void vconv_kernel(logkv_attention_args a, cons
 // Partials of the key-range splits combined in split order: eight queries per
 // block, 32 threads per query, four output features per thread (dv <= 128). A
 // partial's maximum m is of s * scale * log2(e), so a split's weight is
-// 2^(m_split - m).
+// 2^(m_split - m). All splits' loads are issued together: 10 splits of 666 query
+// rows on 8 lanes 5.2 us, one split after the other 10.5 us (2 splits of 2048
+// rows on 16 lanes 12 against 11 us, the price of the 16 predicated loads).
 constexpr int kCombineQueries = 8;
 __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args a, const float* __restrict__ part,
                                                             int splits, const int32_t* __restrict__ vshift) {
@@ -516,19 +515,32 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
   const int qi = blockIdx.x * kCombineQueries + static_cast<int>(threadIdx.x) / 32;
   const int d = 4 * (static_cast<int>(threadIdx.x) % 32);
   if (qi >= nq || d >= a.dv) return;
-  const int stride = a.dv + 2;
+  const int stride = a.dv + kPartTail;
   const float* base = part + (static_cast<int64_t>(lane_ix) * splits * nq + qi) * stride;
   const int64_t step = static_cast<int64_t>(nq) * stride;
+  float2 ml[kMaxChunkSplits];
+  float4 x[kMaxChunkSplits];
   float m = -__builtin_inff();
-  for (int sp = 0; sp < splits; ++sp) m = fmaxf(m, base[sp * step]);
-  float lsum = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int sp = 0; sp < splits; ++sp) {
-    const float* pp = base + sp * step;
-    if (pp[0] == -__builtin_inff()) continue;
-    const float f = __builtin_amdgcn_exp2f(pp[0] - m);   // maxima are in the base-2 domain
-    lsum += pp[1] * f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] += pp[2 + d + j] * f;
+  for (int sp = 0; sp < kMaxChunkSplits; ++sp) {
+    ml[sp] = make_float2(-__builtin_inff(), 0.f);
+    if (sp < splits) {
+      ml[sp] = *reinterpret_cast<const float2*>(base + sp * step + a.dv);
+      x[sp] = *reinterpret_cast<const float4*>(base + sp * step + d);
+    }
+  }
+#pragma unroll
+  for (int sp = 0; sp < kMaxChunkSplits; ++sp) m = fmaxf(m, ml[sp].x);
+  float lsum = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int sp = 0; sp < kMaxChunkSplits; ++sp) {
+    if (sp >= splits || ml[sp].x == -__builtin_inff()) continue;
+    const float f = __builtin_amdgcn_exp2f(ml[sp].x - m);   // maxima are in the base-2 domain
+    lsum += ml[sp].y * f;
+    acc[0] += x[sp].x * f;
+    acc[1] += x[sp].y * f;
+    acc[2] += x[sp].z * f;
+    acc[3] += x[sp].w * f;
   }
   const int head = g * rep + qi / a.tq, t = qi % a.tq;
   // Partials hold 2^(15 - k) sum P V (see chunk_kernel's output).
@@ -546,7 +558,6 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
 // split charged one tile for its start and its partials, never shorter than four
 // tiles of the packed capacity and at most kMaxChunkSplits. 24 query blocks over
 // 2.5K rows: 10 splits 29.6 us, 6 (one per 1024 rows of capacity) 31.6 us.
-constexpr int kMaxChunkSplits = 16;
 int chunk_splits(const logkv_attention_args& a) {
   const int nq = (a.n_heads / a.n_groups) * a.tq;
   const int64_t blocks = static_cast<int64_t>((nq + kQRows - 1) / kQRows) * a.n_batch * a.n_groups;
@@ -585,7 +596,7 @@ static ChunkWs chunk_ws(const logkv_attention_args& a, void* base) {
   int64_t off = 0;
   ChunkWs w{};
   w.part = splits > 1 && b ? reinterpret_cast<float*>(b + off) : nullptr;
-  if (splits > 1) off += align256(lanes * splits * nq * (a.dv + 2) * 4);
+  if (splits > 1) off += align256(lanes * splits * nq * (a.dv + kPartTail) * 4);
   w.vmax = b ? reinterpret_cast<int32_t*>(b + off) : nullptr;
   off += align256(lanes * kVSlices * 2 * 4);
   w.vshift = b ? reinterpret_cast<int32_t*>(b + off) : nullptr;
