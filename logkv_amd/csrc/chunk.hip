@@ -557,13 +557,17 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
 // Key-range splits: the count whose rounds of blocks over the CUs cost least, a
 // split charged one tile for its start and its partials, never shorter than four
 // tiles of the packed capacity and at most kMaxChunkSplits. 24 query blocks over
-// 2.5K rows: 10 splits 29.6 us, 6 (one per 1024 rows of capacity) 31.6 us.
+// 2.5K rows: 10 splits 29.6 us, 6 (one per 1024 rows of capacity) 31.6 us. Below
+// 2048 rows of capacity there is one split: P is rounded relative to a split's
+// own maximum, and a short readout's rounding should not depend on the capacity
+// that its buffer was sized for.
 int chunk_splits(const logkv_attention_args& a) {
   const int nq = (a.n_heads / a.n_groups) * a.tq;
   const int64_t blocks = static_cast<int64_t>((nq + kQRows - 1) / kQRows) * a.n_batch * a.n_groups;
   const int64_t resident = 256 * kBlocksPerCu;
   const int tiles = (a.cap + kKeys - 1) / kKeys;
   int best = 1;
+  if (a.cap < 2048) return best;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= std::min(kMaxChunkSplits, std::max(1, tiles / 4)); ++s) {
     const int64_t cost = (blocks * s + resident - 1) / resident * ((tiles + s - 1) / s + 1) + (s > 1 ? 2 : 0);
