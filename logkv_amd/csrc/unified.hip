@@ -843,6 +843,7 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_plan_kernel(ReduceArgs 
 // LDS instead and a store writes 4 rows x the tile's 16 kept columns, which
 // share cache lines. First round of a 4096-row flush, 32 lanes: 1.21 -> 0.91 ms.
 constexpr int kLwCols = 2, kLwRows = 16, kLwTile = kLwCols * kWave;
+constexpr int kLwStaged = 8;   // merges per item from which the mirrors go through LDS
 constexpr int kLwLd = kLwTile + 4;   // LDS row stride: a store's 16 rows x 4 columns fall into distinct banks
 
 template <bool LIMIT>
@@ -862,6 +863,10 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
   // Merges per item: up to kLwRows, fewer when that would leave waves idle.
   const int rows = max(1, min(kLwRows, n_ok * col_chunks / waves));
   const int items = col_chunks * ((n_ok + rows - 1) / rows);
+  // Items of few merges (a small flush, a late round) write their mirrors as they go: LDS would
+  // only add a pass whose stores have most of their lanes idle (two flushes of 1024 rows over 8
+  // lanes 3.99 ms, 4.24 with every item staged; of 3000 rows over 16 lanes 14.31 and 14.22).
+  const bool staged = rows >= kLwStaged;
   float* tile = tile_s[wave_id()];
   int* mirror = mirror_s[wave_id()];
   for (int it = blockIdx.x * kPhaseWaves + wave_id(); it < items; it += waves) {
@@ -947,7 +952,8 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
         if (c >= 0) {
           row_a[c] = nw[e];
         }
-        tile[j * kLwLd + e * kWave + l] = nw[e];
+        if (staged) tile[j * kLwLd + e * kWave + l] = nw[e];
+        else if (c >= 0 && !(fl[e] & kKeep)) dist[static_cast<int64_t>(c) * M + ra] = nw[e];
         sc[e] = screen_cost<LIMIT>(nw[e], total, mc[e], rad, rc[e], limit, c >= 0 && c != ra, border[e]);
         if (!border[e]) m = sc[e] < m ? sc[e] : m;
       }
@@ -970,6 +976,7 @@ __global__ __launch_bounds__(kPhaseThreads) void reduce_lw_kernel(ReduceArgs a) 
       if (l == 0 && best < kInfKey)
         atomicMin(reinterpret_cast<unsigned long long*>(&s.packed[ra]), static_cast<unsigned long long>(best));
     }
+    if (!staged) continue;
     // The mirrors: lane l writes kept column l % 16 of tile column 4 i + l / 16. The wave's own LDS
     // (its accesses complete in order; the fences keep the compiler's order).
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
