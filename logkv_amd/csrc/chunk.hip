@@ -554,13 +554,19 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
   *reinterpret_cast<LOGKV_G uint2*>(o) = make_uint2(lo, hi);
 }
 
-// Key-range splits: the count whose rounds of blocks over the CUs cost least, a
-// split charged one tile for its start and its partials, never shorter than four
-// tiles of the packed capacity and at most kMaxChunkSplits. 24 query blocks over
-// 2.5K rows: 10 splits 29.6 us, 6 (one per 1024 rows of capacity) 31.6 us. Below
-// 2048 rows of capacity there is one split: P is rounded relative to a split's
-// own maximum, and a short readout's rounding should not depend on the capacity
-// that its buffer was sized for.
+// Key-range splits: the count that costs least, at most kMaxChunkSplits and never shorter than four
+// tiles of the packed capacity. The unit is a block's tile (2.3 us at 128 features, 1.4 us at 64):
+//  * rounds of blocks over the CUs, each of a split's tiles and one more for its start;
+//  * with more than one split, two tiles for the combine launch and 1/32 tile for every block's
+//    float32 partials, written and read back (256 rows, 0.14 MB at 128 features; 0.5 to 0.6 us per
+//    MB). Without that charge 480 query blocks over 12K rows took 9 splits to save four tiles and
+//    moved 1.2 GB for them: 1234 us, with one split 883 us (272 blocks: 10 splits 732 us, 4 648 us).
+// Few blocks gain from many splits: 24 over 2.5K rows 38 us with 9, 55 us with 2, 81 us with 1.
+// P is rounded relative to a split's own running maximum, so outputs of different counts differ
+// within P's fp16 rounding; the count follows the capacity of the packed buffer, the host's only
+// bound on its rows. Below 2048 rows of capacity there is one split whatever it costs (two lanes of
+// 40 query rows over 1.9K: 76 us, 28 us with 7): the outputs over such a buffer are one online
+// softmax's, bit for bit what they were before longer ranges were split more often.
 int chunk_splits(const logkv_attention_args& a) {
   const int nq = (a.n_heads / a.n_groups) * a.tq;
   const int64_t blocks = static_cast<int64_t>((nq + kQRows - 1) / kQRows) * a.n_batch * a.n_groups;
@@ -568,9 +574,10 @@ int chunk_splits(const logkv_attention_args& a) {
   const int tiles = (a.cap + kKeys - 1) / kKeys;
   int best = 1;
   if (a.cap < 2048) return best;
-  int64_t best_cost = INT64_MAX;
+  int64_t best_cost = INT64_MAX;   // in 1/32 tiles
   for (int s = 1; s <= std::min(kMaxChunkSplits, std::max(1, tiles / 4)); ++s) {
-    const int64_t cost = (blocks * s + resident - 1) / resident * ((tiles + s - 1) / s + 1) + (s > 1 ? 2 : 0);
+    const int64_t rounds = (blocks * s + resident - 1) / resident;
+    const int64_t cost = 32 * rounds * ((tiles + s - 1) / s + 1) + (s > 1 ? 64 + blocks * s : 0);
     if (cost < best_cost) {
       best_cost = cost;
       best = s;
