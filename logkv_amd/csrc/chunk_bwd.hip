@@ -30,8 +30,9 @@
 // Measured at 2 x 1024 query rows, 16 heads of 128 on 8 groups, 9.3K packed rows and a 1024-row
 // chunk: dq 264 us and statistics 185 us (one 128-row block of four waves, tiles staged by element
 // and re-read from LDS as both operands: 1880 us together), dk / dv 99 us with its rows loaded as
-// 16-byte units (1224 us by element); bound by matrix-core issue and the exponentials of the two
-// waves of a SIMD running in step.
+// 16-byte units (1224 us by element); dq and statistics bound by the matrix products and the
+// exponentials, which the two waves of a SIMD run in step and so one after the other; dk / dv, one
+// wave per SIMD, by the latency of that same chain (matrix cores 22% busy).
 #include <algorithm>
 
 #include "route.hpp"
@@ -629,14 +630,19 @@ __global__ __launch_bounds__(256) void sum_dkv_kernel(logkv_attention_args a, lo
 
 namespace {
 
-// Parts of a walk of `tiles` tiles for `blocks` blocks at one block per CU: the count whose
-// rounds over the 256 CUs cost least, each part charged one tile for its start and partials.
+// Parts of a walk of `tiles` tiles for `blocks` blocks at one block per CU: the count that costs
+// least in tiles (dq and statistics together 6.4 us, dk / dv 5.3 us at 128 features): rounds over
+// the 256 CUs, each of a part's tiles and one more for its start, and with more than one part a tile
+// for the summing launch and 1/128 tile for every block's float32 partials, written and read back
+// (0.13 MB at 128 features; at 1/64 a 512-row chunk of 8 lanes lost parts that pay, 99 -> 104 us). Without that charge 480 query blocks over 12K rows took 9 parts and
+// 570 MB of partials to save three tiles: 3111 us, with one part 2908 us (288 over 5K: 8 parts 982,
+// 5 parts 866 us).
 int bwd_splits(int64_t blocks, int tiles) {
   int best = 1;
-  double best_cost = 1e30;
+  int64_t best_cost = INT64_MAX;   // in 1/128 tiles
   for (int s = 1; s <= std::min(kMaxSplits, std::max(1, tiles / 2)); ++s) {
-    const double rounds = static_cast<double>((blocks * s + 255) / 256);
-    const double cost = rounds * ((tiles + s - 1) / s + 1) + (s > 1 ? 1 : 0);
+    const int64_t rounds = (blocks * s + 255) / 256;
+    const int64_t cost = 128 * rounds * ((tiles + s - 1) / s + 1) + (s > 1 ? 128 + blocks * s : 0);
     if (cost < best_cost) {
       best_cost = cost;
       best = s;

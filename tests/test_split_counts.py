@@ -33,6 +33,16 @@ def forward_splits(batch, groups, heads, tq, dim, cap):
     return max(1, round(part / (lanes * nq * (dim + 4) * 4)))
 
 
+def backward_parts(batch, groups, heads, tq, dim, cap):
+    """Parts of the key range in the backward, from the statistics' partials and dq's (dq's the larger
+    of the two gradients here)."""
+    lanes, nq = batch * groups, heads // groups * tq
+    a = _args(batch, groups, heads, tq, dim, cap)
+    floats = _lib.lib().logkv_chunk_backward_workspace_bytes(C.byref(a)) / 4 - lanes * nq * 2
+    one = lanes * nq * 4
+    return 1 if floats < lanes * nq * dim else round(floats / (one + lanes * nq * dim))
+
+
 @pytest.mark.parametrize("shape,fast", [
     ((2, 8, 32, 1920, 128, 12000), {1}),            # 1: 883, 2: 961, 4: 1030, 9: 1229
     ((2, 8, 24, 1400, 128, 12000), {3, 4, 5}),      # 1: 848, 2: 698, 3: 656, 4: 652, 5: 650, 7: 681, 10: 748
@@ -47,3 +57,15 @@ def forward_splits(batch, groups, heads, tq, dim, cap):
 ])
 def test_forward_takes_a_fast_count(shape, fast):
     assert forward_splits(*shape) in fast
+
+
+@pytest.mark.parametrize("shape,fast", [
+    ((2, 8, 32, 1920, 128, 12000), {1, 2}),         # 1: 2907, 2: 2942, 4: 2982, 9: 3098
+    ((2, 8, 32, 1100, 128, 5000), {3, 4, 5}),       # 1: 1104, 2: 909, 3: 862, 4: 857, 5: 880, 8: 967
+    ((2, 8, 24, 1400, 128, 12000), {4, 5, 6, 7, 8}),   # 1: 2459, 2: 1906, 4: 1711, 5: 1663, 6: 1666, 8: 1682, 10: 1735
+    ((2, 8, 16, 1024, 128, 13000), {2}),            # 1: 1004, 2: 599, 4: 628
+    ((1, 8, 16, 333, 128, 4000), {8, 9}),           # 1: 326, 2: 188, 4: 123, 8: 97, 9: 95
+    ((1, 8, 8, 64, 128, 19000), {16}),              # 1: 1557, 8: 235, 16: 145
+])
+def test_backward_takes_a_fast_count(shape, fast):
+    assert backward_parts(*shape) in fast
