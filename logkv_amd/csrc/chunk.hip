@@ -115,9 +115,10 @@ __device__ __forceinline__ ChunkBlock chunk_block() {
 // s-th of `splits` equal parts (whole 64-row tiles) of its queries' key range
 // and writes partials [acc[dv], m, l, 0, 0] per query (m in the base-2 domain).
 // NKS 16-wide steps of the packed width and NDV 32-wide blocks of dv at
-// compile time (straight-line tile code); columns past the packed width and
-// V columns past dv are zero, so a kernel with more steps or blocks than the
-// shape needs gives the same result.
+// compile time (straight-line tile code); columns past the packed width are
+// zero, and V columns past dv reach only accumulators that are not written out,
+// so a kernel with more steps or blocks than the shape needs gives the same
+// result.
 // BF16V: the body of a lane without an exact fp16 V copy (vshift kBf16Lane).
 template <int NKS, int NDV, bool BF16V>
 __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const int32_t* __restrict__ width_ptr,
@@ -182,7 +183,9 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
   const int vstride = BF16V ? dim : a.dv;
   const int units = dim / 8;
   // Each thread's staging tasks are the same in every tile: up to kKTasks
-  // 16-byte K units and kVTasks V units (row, unit; zero past dv).
+  // 16-byte K units and kVTasks V units (row, unit). V units past dv are neither
+  // loaded nor stored (dv 96 in the full kernel: 2000 rows of 16 heads over 15K
+  // rows 306 us, with zeros staged there 362 us).
   constexpr int kUnitsV = 4 * NDV;
   constexpr int kKTasks = (kKeys * kMaxSteps * 2 + kThreads - 1) / kThreads, kVTasks = kKeys * kUnitsV / kThreads;
   int k_row[kKTasks], k_goff[kKTasks], k_loff[kKTasks];
@@ -208,9 +211,8 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
 #pragma unroll
     for (int q = 0; q < kVTasks; ++q) {
       const int i = threadIdx.x + kThreads * q, r = i / kUnitsV, u = i % kUnitsV;
-      const bool on = r < rows && 8 * u < a.dv;
-      vx[q] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + (on ? r : 0)) * vstride + (on ? 8 * u : 0));
-      if (!on) vx[q] = make_uint4(0, 0, 0, 0);
+      if (8 * u < a.dv) vx[q] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + min(r, rows - 1)) * vstride + 8 * u);
+      if (r >= rows) vx[q] = make_uint4(0, 0, 0, 0);
     }
   };
   // Both row-major; rows past the end are zeros.
@@ -220,8 +222,8 @@ __device__ __forceinline__ void chunk_body(const logkv_attention_args& a, const 
       if (k_row[q] < kKeys) *reinterpret_cast<uint4*>(&k_s[bf][k_loff[q]]) = kx[q];
 #pragma unroll
     for (int q = 0; q < kVTasks; ++q) {
-      const int i = threadIdx.x + kThreads * q;
-      *reinterpret_cast<uint4*>(&v_s[bf][(i / kUnitsV) * kLdV + 8 * (i % kUnitsV)]) = vx[q];
+      const int i = threadIdx.x + kThreads * q, r = i / kUnitsV, u = i % kUnitsV;
+      if (8 * u < a.dv) *reinterpret_cast<uint4*>(&v_s[bf][r * kLdV + 8 * u]) = vx[q];
     }
   };
   const int ntiles = k_begin < k_stop ? (k_stop - k_begin + kKeys - 1) / kKeys : 0;
@@ -629,7 +631,7 @@ int launch_chunk_attention(const logkv_attention_args& a, const int32_t* width, 
   hipLaunchKernelGGL(vmax_kernel, vgrid, dim3(256), 0, stream, a, width, w.vmax);
   hipLaunchKernelGGL(vconv_kernel, vgrid, dim3(256), 0, stream, a, width, w.vmax, w.vshift, w.v16);
   // Shapes with at most 5 steps and 2 dv blocks (head dim 64) take the
-  // smaller kernel; every other shape runs the full 9 x 4 one on zero padding.
+  // smaller kernel; every other shape runs the full 9 x 4 one.
   if (a.dim <= 80 && a.dv <= 64)
     hipLaunchKernelGGL((chunk_kernel<5, 2>), grid, dim3(kThreads), 0, stream, a, width, splits, w.part, w.v16,
                        w.vshift);

@@ -634,9 +634,9 @@ namespace {
 // least in tiles (dq and statistics together 6.4 us, dk / dv 5.3 us at 128 features): rounds over
 // the 256 CUs, each of a part's tiles and one more for its start, and with more than one part a tile
 // for the summing launch and 1/128 tile for every block's float32 partials, written and read back
-// (0.13 MB at 128 features; at 1/64 a 512-row chunk of 8 lanes lost parts that pay, 99 -> 104 us). Without that charge 480 query blocks over 12K rows took 9 parts and
-// 570 MB of partials to save three tiles: 3111 us, with one part 2908 us (288 over 5K: 8 parts 982,
-// 5 parts 866 us).
+// (0.13 MB at 128 features; at 1/64 a 512-row chunk of 8 lanes lost parts that pay, 99 -> 104 us).
+// Without that charge 480 query blocks over 12K rows took 9 parts and 570 MB of partials to save
+// three tiles: 3111 us, with one part 2908 us (288 over 5K: 8 parts 982, 5 parts 866 us).
 int bwd_splits(int64_t blocks, int tiles) {
   int best = 1;
   int64_t best_cost = INT64_MAX;   // in 1/128 tiles

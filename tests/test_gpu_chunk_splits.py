@@ -29,6 +29,8 @@ pytestmark = pytest.mark.gpu
     (1, 8, 32, 1000, 128, 900, 2100, 2),
     (1, 2, 2, 40, 128, 2000, 2047, 1),
     (1, 2, 2, 40, 128, 2000, 2048, 8),
+    (1, 2, 2, 70, 32, 300, 400, 1),           # values of half the narrow kernel's width
+    (2, 2, 4, 300, 96, 5000, 6000, 16),       # values of three quarters of the full kernel's
 ])
 def test_split_counts_match_float64(batch, groups, heads, tq, dim, rows, cap, splits):
     assert forward_splits(batch, groups, heads, tq, dim, cap) == splits
