@@ -505,10 +505,13 @@ __global__ __launch_bounds__(256) void vconv_kernel(logkv_attention_args a, cons
 // Partials of the key-range splits combined in split order: eight queries per
 // block, 32 threads per query, four output features per thread (dv <= 128). A
 // partial's maximum m is of s * scale * log2(e), so a split's weight is
-// 2^(m_split - m). All splits' loads are issued together: 10 splits of 666 query
-// rows on 8 lanes 5.2 us, one split after the other 10.5 us (2 splits of 2048
-// rows on 16 lanes 12 against 11 us, the price of the 16 predicated loads).
+// 2^(m_split - m). All splits' loads are issued together, in a kernel for up to
+// MAX of them: 10 splits of 666 query rows on 8 lanes 5.2 us (one split after the
+// other 10.5 us); 2 splits of 4096 query rows on 8 lanes 9.4 us with loads for 4,
+// 11.9 us with loads for 16 (one after the other 10.5 us).
 constexpr int kCombineQueries = 8;
+constexpr int kFewSplits = 4;
+template <int MAX>
 __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args a, const float* __restrict__ part,
                                                             int splits, const int32_t* __restrict__ vshift) {
   const int lane_ix = blockIdx.y, G = a.n_groups;
@@ -520,11 +523,11 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
   const int stride = a.dv + kPartTail;
   const float* base = part + (static_cast<int64_t>(lane_ix) * splits * nq + qi) * stride;
   const int64_t step = static_cast<int64_t>(nq) * stride;
-  float2 ml[kMaxChunkSplits];
-  float4 x[kMaxChunkSplits];
+  float2 ml[MAX];
+  float4 x[MAX];
   float m = -__builtin_inff();
 #pragma unroll
-  for (int sp = 0; sp < kMaxChunkSplits; ++sp) {
+  for (int sp = 0; sp < MAX; ++sp) {
     ml[sp] = make_float2(-__builtin_inff(), 0.f);
     if (sp < splits) {
       ml[sp] = *reinterpret_cast<const float2*>(base + sp * step + a.dv);
@@ -532,10 +535,10 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(logkv_attention_args
     }
   }
 #pragma unroll
-  for (int sp = 0; sp < kMaxChunkSplits; ++sp) m = fmaxf(m, ml[sp].x);
+  for (int sp = 0; sp < MAX; ++sp) m = fmaxf(m, ml[sp].x);
   float lsum = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int sp = 0; sp < kMaxChunkSplits; ++sp) {
+  for (int sp = 0; sp < MAX; ++sp) {
     if (sp >= splits || ml[sp].x == -__builtin_inff()) continue;
     const float f = __builtin_amdgcn_exp2f(ml[sp].x - m);   // maxima are in the base-2 domain
     lsum += ml[sp].y * f;
@@ -638,9 +641,13 @@ int launch_chunk_attention(const logkv_attention_args& a, const int32_t* width, 
   else
     hipLaunchKernelGGL((chunk_kernel<kMaxSteps, kMaxDvBlocks>), grid, dim3(kThreads), 0, stream, a, width, splits,
                        w.part, w.v16, w.vshift);
-  if (splits > 1)
-    hipLaunchKernelGGL(chunk_combine_kernel, dim3((nq + kCombineQueries - 1) / kCombineQueries, a.n_batch * a.n_groups),
-                       dim3(256), 0, stream, a, w.part, splits, w.vshift);
+  if (splits > 1) {
+    const dim3 cgrid((nq + kCombineQueries - 1) / kCombineQueries, a.n_batch * a.n_groups);
+    if (splits <= kFewSplits)
+      hipLaunchKernelGGL(chunk_combine_kernel<kFewSplits>, cgrid, dim3(256), 0, stream, a, w.part, splits, w.vshift);
+    else
+      hipLaunchKernelGGL(chunk_combine_kernel<kMaxChunkSplits>, cgrid, dim3(256), 0, stream, a, w.part, splits, w.vshift);
+  }
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }
 

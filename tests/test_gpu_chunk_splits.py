@@ -30,6 +30,8 @@ pytestmark = pytest.mark.gpu
     (1, 2, 2, 40, 128, 2000, 2047, 1),
     (1, 2, 2, 40, 128, 2000, 2048, 8),
     (1, 2, 2, 70, 32, 300, 400, 1),           # values of half the narrow kernel's width
+    (2, 8, 8, 1024, 128, 3900, 4000, 4),     # the most splits that the combine for few of them takes
+    (2, 4, 16, 333, 64, 6000, 6600, 5),       # and one more
     (2, 2, 4, 300, 96, 5000, 6000, 16),       # values of three quarters of the full kernel's
 ])
 def test_split_counts_match_float64(batch, groups, heads, tq, dim, rows, cap, splits):
