@@ -40,7 +40,7 @@ constexpr int v_stride(int blocks) { return 16 * blocks + 16; }
 
 // NS 32-wide steps of the packed width, NB 16-wide blocks of dv.
 template <int NS, int NB>
-__global__ __launch_bounds__(64 * kWaves, NS <= 5 ? 2 : 1) void decode_mfma_kernel(logkv_attention_args a,
+__global__ __launch_bounds__(64 * kWaves, NB <= 8 ? 2 : 1) void decode_mfma_kernel(logkv_attention_args a,
                                                                      const int32_t* __restrict__ width_ptr,
                                                                      float* __restrict__ part) {
   typedef __attribute__((address_space(3))) s16x4* lds4;
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(64 * kWaves, NS <= 5 ? 2 : 1) void decode_mfma_kern
   __shared__ __align__(16) uint8_t buf[kWaves][kTileBytes > kOutBytes ? kTileBytes : kOutBytes];
   __shared__ float m_s[kWaves][kQ], l_s[kWaves][kQ];
   const int lane = blockIdx.y, G = a.n_groups, b = lane / G, g = lane % G;
-  const int rep = a.n_heads / G, nq = rep * a.tq, dim = a.dim, units = dim / 8;
+  const int rep = a.n_heads / G, nq = rep * a.tq, dim = a.dim, units = dim / 8, vunits = (a.dv + 7) / 8;
   const int w = wave_id(), l = lane_id(), col = l & 15, hq = l >> 4;
   const int total = min(*width_ptr + a.tail + (a.alpha_count_dev ? *a.alpha_count_dev : 0), a.cap);
   const int tail0 = total - a.causal_tail;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * kWaves, NS <= 5 ? 2 : 1) void decode_mfma_kern
     for (int i = 0; i < kVLoads; ++i) {
       const int e = l + 64 * i, r = e / (2 * NB), u = e % (2 * NB);
       vx[i] = make_uint4(0, 0, 0, 0);
-      if (u < units && t0 + r < r_end) vx[i] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + r) * dim + 8 * u);
+      if (u < vunits && t0 + r < r_end) vx[i] = *(const LOGKV_G uint4*)(vbase + static_cast<int64_t>(t0 + r) * dim + 8 * u);
     }
   };
   f32x4 o[NB];
@@ -234,13 +234,16 @@ __global__ __launch_bounds__(64 * kWaves, NS <= 5 ? 2 : 1) void decode_mfma_kern
 
 int launch_decode_mfma(const logkv_attention_args& a, const int32_t* width, float* part, int n_split, hipStream_t stream) {
   const dim3 grid(n_split, a.n_batch * a.n_groups);
-  // Head dims up to 64 and up to 128 have kernels of their own (registers for four and two waves
-  // per SIMD); wider rows, up to the packed limit of 264 and dv of 256, take the full one. Units
-  // a shape does not have are zero.
+  // By packed width and value width: head dims up to 64 and up to 128, wider keys with values up to
+  // 128 (all at two waves per SIMD), and the rest up to the packed limit of 264 and dv of 256 (one).
+  // Units a shape does not have are zero and not read. Keys of 192 with values of 128, 64 lanes of 4K
+  // rows, 2 queries: 40 us (47 us in the widest kernel, which also read the values' padding).
   if (a.dim <= 96 && a.dv <= 64)
     hipLaunchKernelGGL((decode_mfma_kernel<3, 4>), grid, dim3(64 * kWaves), 0, stream, a, width, part);
   else if (a.dim <= 160 && a.dv <= 128)
     hipLaunchKernelGGL((decode_mfma_kernel<5, 8>), grid, dim3(64 * kWaves), 0, stream, a, width, part);
+  else if (a.dv <= 128)
+    hipLaunchKernelGGL((decode_mfma_kernel<9, 8>), grid, dim3(64 * kWaves), 0, stream, a, width, part);
   else
     hipLaunchKernelGGL((decode_mfma_kernel<9, 16>), grid, dim3(64 * kWaves), 0, stream, a, width, part);
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;

@@ -516,10 +516,10 @@ int launch_pack(const logkv_readout_view& c, const logkv_pack_args& p, const int
 }
 
 // Splits per lane: at most one per 128 rows (a 32-row tile for each of a block's four waves), and
-// no more than keep every block of the launch resident (two per CU; one for packed widths above
-// 160). 64 lanes of 8.4K rows of 128 features: 51 us at 512 blocks, 58 at 768, 57 at 1024.
+// no more than keep every block of the launch resident (two per CU; one for values wider than
+// 128). 64 lanes of 8.4K rows of 128 features: 51 us at 512 blocks, 58 at 768, 57 at 1024.
 int attention_splits(const logkv_attention_args& a) {
-  const int lanes = a.n_batch * a.n_groups, blocks = a.dim <= 160 && a.dv <= 128 ? 512 : 256;
+  const int lanes = a.n_batch * a.n_groups, blocks = a.dv <= 128 ? 512 : 256;
   return std::max(1, std::min((a.cap + 127) / 128, blocks / std::max(1, lanes)));
 }
 

@@ -31,6 +31,8 @@ CASES = [
     (1, 1, 2, 1, 192, 128, 700, 1),
     (1, 1, 4, 2, 256, 256, 400, 2),
     (40, 16, 16, 1, 64, 64, 200, 1),
+    (64, 4, 8, 1, 192, 128, 700, 1),        # 2 splits of three passes
+    (1, 2, 4, 2, 168, 100, 300, 2),
 ]
 
 
