@@ -6,7 +6,8 @@
 // Bf16 rows move in 16-byte units of eight features (8-byte ones where a width
 // or a source row does not allow it), one per thread, a block per 256 units of
 // one lane's buffer, so that a block's source and destination are uniform;
-// positions and span flags one entry per thread. Bound by HBM: 224 lanes x 2048
+// positions and span flags one entry per thread. A launch holds at most 2^31
+// threads; longer moves are several launches. Bound by HBM: 224 lanes x 2048
 // rows of 3 x 128 features are appended in 159 us (4.4 TB/s; 8-byte units in a
 // grid-stride loop over all buffers 191 us; two units per thread 164 us, and
 // 18 us instead of 7 us at 8 lanes) and moved and cleared in 183 us (239 us).
@@ -19,6 +20,7 @@ namespace logkv {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int64_t kLaunchThreads = int64_t(1) << 31;   // threads of one launch
 
 template <int F>
 struct UnitOf;
@@ -37,18 +39,19 @@ struct UnitOf<8> {
 struct RowBlock {
   int lane, buf, first;
 };
-__device__ __forceinline__ RowBlock row_block(int chunks) {
+__device__ __forceinline__ RowBlock row_block(int chunks, int lane0) {
   const int i = static_cast<int>(blockIdx.x) / chunks;
-  return RowBlock{i / 3, i % 3, (static_cast<int>(blockIdx.x) - i * chunks) * kThreads};
+  return RowBlock{lane0 + i / 3, i % 3, (static_cast<int>(blockIdx.x) - i * chunks) * kThreads};
 }
 
 }  // namespace
 
-// Block rows [0, n) of each source into recent rows [at, at + n); `chunks` blocks to a lane's buffer.
+// Rows [0, n) of each source into recent rows [at, at + n); `chunks` blocks to a lane's buffer.
 template <int F>
-__global__ __launch_bounds__(kThreads) void recent_append_kernel(logkv_recent_args a, int at, int n, int chunks) {
+__global__ __launch_bounds__(kThreads) void recent_append_kernel(logkv_recent_args a, int at, int n, int chunks,
+                                                                    int lane0) {
   using Unit = typename UnitOf<F>::type;
-  const RowBlock blk = row_block(chunks);
+  const RowBlock blk = row_block(chunks, lane0);
   const int b = blk.lane / a.n_groups, g = blk.lane % a.n_groups, tid = static_cast<int>(threadIdx.x);
   const int d = blk.buf == 0 ? a.dk : (blk.buf == 1 ? a.dkr : a.dv), units = d / F, total = n * units;
   const LOGKV_G uint16_t* src = blk.buf == 0 ? gp(a.k) + b * a.k_sb + g * a.k_sg
@@ -70,21 +73,20 @@ __global__ __launch_bounds__(kThreads) void recent_append_kernel(logkv_recent_ar
   }
 }
 
-// Rows [take, count) move to [0, count - take) and rows [count - take, count)
-// become zero. Needs count - take <= take: then every source row lies in the
-// cleared range, and the thread that reads it clears it.
+// Rows [0, n): the first `remaining` receive the rows `take` further on, which become zero, and the
+// others become zero. Of a window of `count` rows that loses `take` all rows [0, take) are given,
+// with count - take of them receiving: count - take <= take, so every source row lies in the
+// cleared range past them, and the thread that reads it clears it.
 template <int F>
-__global__ __launch_bounds__(kThreads) void recent_shift_kernel(logkv_recent_args a, int take, int count, int chunks) {
+__global__ __launch_bounds__(kThreads) void recent_shift_kernel(logkv_recent_args a, int take, int n, int remaining,
+                                                                   int chunks, int lane0) {
   using Unit = typename UnitOf<F>::type;
-  const RowBlock blk = row_block(chunks);
-  const int remaining = count - take;
+  const RowBlock blk = row_block(chunks, lane0);
   const int b = blk.lane / a.n_groups, g = blk.lane % a.n_groups, tid = static_cast<int>(threadIdx.x);
-  const int d = blk.buf == 0 ? a.dk : (blk.buf == 1 ? a.dkr : a.dv), units = d / F, total = take * units;
+  const int d = blk.buf == 0 ? a.dk : (blk.buf == 1 ? a.dkr : a.dv), units = d / F, total = n * units;
   LOGKV_G uint16_t* dst = (blk.buf == 0 ? gp(a.recent_k) : (blk.buf == 1 ? gp(a.recent_k_raw) : gp(a.recent_v))) +
                           static_cast<int64_t>(blk.lane) * a.cap * d;
   LOGKV_G uint16_t* src = dst + static_cast<int64_t>(take) * d;
-  // Units of rows [0, take): one of the first `remaining` rows receives row
-  // take + r (and clears it); the others are cleared.
   const int moved = remaining * units;
   const int i = blk.first + tid;
   if (i < moved) {
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(kThreads) void recent_shift_kernel(logkv_recent_arg
   }
   if (g != 0 || blk.buf != 0) return;
   const int64_t pos0 = static_cast<int64_t>(b) * a.cap;
-  for (int r = blk.first + tid; r < take; r += chunks * kThreads) {
+  for (int r = blk.first + tid; r < n; r += chunks * kThreads) {
     if (r < remaining) {
       a.recent_pos[pos0 + r] = a.recent_pos[pos0 + take + r];
       a.recent_pos[pos0 + take + r] = 0;
@@ -122,30 +124,53 @@ bool wide_window(const logkv_recent_args& a) {
          rows16(a.recent_k_raw, 0, 0, 0) && rows16(a.recent_v, 0, 0, 0);
 }
 
-template <class Kernel>
-void launch_rows(Kernel kernel, const logkv_recent_args& a, int f, int rows, int first, int second, hipStream_t stream) {
-  const int units = rows * (std::max(a.dk, std::max(a.dkr, a.dv)) / f);
-  const int chunks = (units + kThreads - 1) / kThreads;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(chunks) * 3 * a.n_batch * a.n_groups), dim3(kThreads), 0, stream,
-                     a, first, second, chunks);
+// Calls launch(first row, rows, first lane, grid, chunks) for rows [0, rows) and every lane, in as many
+// parts as kLaunchThreads asks for (one, short of tens of GB).
+template <class Launch>
+void by_parts(const logkv_recent_args& a, int f, int rows, Launch launch) {
+  const int units = std::max(a.dk, std::max(a.dkr, a.dv)) / f;   // of a row's widest buffer
+  const int lanes = a.n_batch * a.n_groups;
+  const int max_rows = static_cast<int>((kLaunchThreads / 3 - kThreads) / units);
+  for (int row0 = 0; row0 < rows; row0 += std::min(max_rows, rows - row0)) {
+    const int n = std::min(max_rows, rows - row0), total = n * units;
+    const int chunks = (total + kThreads - 1) / kThreads;
+    const int max_lanes = static_cast<int>(std::min<int64_t>(lanes, kLaunchThreads / (int64_t(3) * chunks * kThreads)));
+    for (int lane0 = 0; lane0 < lanes; lane0 += std::min(max_lanes, lanes - lane0))
+      launch(row0, n, lane0, dim3(static_cast<unsigned>(chunks) * 3 * std::min(max_lanes, lanes - lane0)), chunks);
+  }
 }
 
 }  // namespace
 
 int launch_recent_append(const logkv_recent_args& a, int at, int n, hipStream_t stream) {
-  if (wide_window(a) && rows16(a.k, a.k_sb, a.k_sg, a.k_st) && rows16(a.k_raw, a.kr_sb, a.kr_sg, a.kr_st) &&
-      rows16(a.v, a.v_sb, a.v_sg, a.v_st))
-    launch_rows(recent_append_kernel<8>, a, 8, n, at, n, stream);
-  else
-    launch_rows(recent_append_kernel<4>, a, 4, n, at, n, stream);
+  const bool wide = wide_window(a) && rows16(a.k, a.k_sb, a.k_sg, a.k_st) && rows16(a.k_raw, a.kr_sb, a.kr_sg, a.kr_st) &&
+                    rows16(a.v, a.v_sb, a.v_sg, a.v_st);
+  by_parts(a, wide ? 8 : 4, n, [&](int row0, int rows, int lane0, dim3 grid, int chunks) {
+    logkv_recent_args p = a;
+    p.k += row0 * a.k_st;
+    p.k_raw += row0 * a.kr_st;
+    p.v += row0 * a.v_st;
+    p.pos += row0 * a.pos_st;
+    if (p.ends) p.ends += row0;
+    hipLaunchKernelGGL(wide ? recent_append_kernel<8> : recent_append_kernel<4>, grid, dim3(kThreads), 0, stream, p,
+                       at + row0, rows, chunks, lane0);
+  });
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }
 
 int launch_recent_shift(const logkv_recent_args& a, int take, int count, hipStream_t stream) {
-  if (wide_window(a))
-    launch_rows(recent_shift_kernel<8>, a, 8, take, take, count, stream);
-  else
-    launch_rows(recent_shift_kernel<4>, a, 4, take, take, count, stream);
+  const bool wide = wide_window(a);
+  by_parts(a, wide ? 8 : 4, take, [&](int row0, int rows, int lane0, dim3 grid, int chunks) {
+    logkv_recent_args p = a;
+    p.recent_k += static_cast<int64_t>(row0) * a.dk;
+    p.recent_k_raw += static_cast<int64_t>(row0) * a.dkr;
+    p.recent_v += static_cast<int64_t>(row0) * a.dv;
+    p.recent_pos += row0;
+    if (p.recent_ends) p.recent_ends += row0;
+    const int remaining = std::max(0, std::min(count - take - row0, rows));
+    hipLaunchKernelGGL(wide ? recent_shift_kernel<8> : recent_shift_kernel<4>, grid, dim3(kThreads), 0, stream, p, take,
+                       rows, remaining, chunks, lane0);
+  });
   return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
 }
 
