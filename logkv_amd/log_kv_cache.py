@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes as C
+import functools
 import math
 from typing import NamedTuple
 
@@ -100,13 +101,13 @@ class _SemanticReplayUpdates:
 
 class _HostOpLog:
     """A finished op-log's rows on the host: ``rows`` int32 ``[Bt, G, max_len, 4]`` and ``lengths``
-    ``[Bt, G]``, both copies. Row tuples are built where they are read (``lists()``, indexing): a
-    training step over 4096 tokens keeps 30K rows that only a failed check would ever print."""
+    ``[Bt, G]``, copies that nothing writes. The row tuples that callers see are built from it on first
+    read: a training step over 4096 tokens logs 30K rows and reads none of them on the host."""
 
-    __slots__ = ("_rows", "_lengths", "_frozen")
+    __slots__ = ("_rows", "_lengths")
 
     def __init__(self, rows, lengths):
-        self._rows, self._lengths, self._frozen = rows, lengths, None
+        self._rows, self._lengths = rows, lengths
 
     def lists(self):
         """Fresh ``[Bt][G]`` lists of (op, cluster, arg, position) tuples."""
@@ -114,36 +115,37 @@ class _HostOpLog:
         return [[list(map(tuple, lane[:n].tolist())) for lane, n in zip(batch, row)]
                 for batch, row in zip(self._rows, lens)]
 
-    def _tuples(self):
-        if self._frozen is None:
-            self._frozen = tuple(tuple(map(tuple, batch)) for batch in self.lists())
-        return self._frozen
-
-    def __len__(self):
-        return self._rows.size(0)
-
-    def __getitem__(self, i):
-        return self._tuples()[i]
-
-    def __iter__(self):
-        return iter(self._tuples())
-
 
 class _SemanticReplayPlans:
     """Host-only replay state of one invocation (litgpt/log_kv_cache.py:97-108).
 
-    Freezes the CPU op-log so later caller mutations cannot change it, and
-    remembers the flush positions seen at each replay cursor, so a replay with
-    different positions at the same cursor is rejected. The log itself is
-    parsed on the device; this object holds no tensors and no cache reference.
+    Freezes the CPU op-log so later caller mutations cannot change it
+    (``host_log``, nested tuples; built on first read from a ``_HostOpLog``,
+    which cannot change), and remembers the flush positions seen at each
+    replay cursor, so a replay with different positions at the same cursor is
+    rejected. The log itself is parsed on the device; this object holds no
+    device tensors and no cache reference.
     """
 
     def __init__(self, host_log):
         if host_log is None:
             raise RuntimeError("semantic replay plans require an existing CPU op-log")
-        self.host_log = (host_log if isinstance(host_log, _HostOpLog) else
-                         tuple(tuple(tuple(map(tuple, lane)) for lane in batch) for batch in host_log))
+        self._source = host_log if isinstance(host_log, _HostOpLog) else None
+        if self._source is None:
+            self.host_log = self._freeze(host_log)
         self.plans = {}
+
+    @staticmethod
+    def _freeze(host_log):
+        return tuple(tuple(tuple(map(tuple, lane)) for lane in batch) for batch in host_log)
+
+    @functools.cached_property
+    def host_log(self):
+        return self._freeze(self._source.lists())
+
+    def holds(self, host_log) -> bool:
+        """Whether ``host_log`` is this object's log: its ``host_log``, or what that is built from."""
+        return host_log is not None and (host_log is self._source or host_log is self.__dict__.get("host_log"))
 
 
 class LogStructuredKVCache(nn.Module):
@@ -419,7 +421,7 @@ class LogStructuredKVCache(nn.Module):
         self.op_log: torch.Tensor | None = None
         self.op_log_len: torch.Tensor | None = None
         self._op_replay_cursor_host = None
-        self._op_log_host = self._op_log_lists = None
+        self._last_op_log_host = None
         # Update tape (semantic_replay_updates): the bound tape, whether it is
         # replayed, and the flushes recorded / replayed since the log began.
         self._active_updates = None
@@ -784,16 +786,21 @@ class LogStructuredKVCache(nn.Module):
         if int(lengths.max()) > self.op_log.size(2):
             raise RuntimeError("semantic LogKV op_log overflow")
         max_len = int(lengths.max())
-        self._op_log_host = _HostOpLog(self.op_log[:, :, :max_len].cpu(), lengths)
-        self._op_log_lists = None
+        self._last_op_log_host = _HostOpLog(self.op_log[:, :, :max_len].cpu(), lengths)
         return self.op_log[:, :, :max_len].clone(), self.op_log_len.clone()
 
     @property
     def _last_op_log_host(self):
-        """``[Bt][G]`` lists of the last taken log's row tuples (None before any); built on first read."""
-        if self._op_log_host is not None and self._op_log_lists is None:
-            self._op_log_lists = self._op_log_host.lists()
-        return self._op_log_lists
+        """``[Bt][G]`` lists of the last taken log's row tuples (None before any); built on first read
+        and the caller's from then on."""
+        log = self.__dict__.get("_last_op_log_host")
+        if isinstance(log, _HostOpLog):
+            log = self.__dict__["_last_op_log_host"] = log.lists()
+        return log
+
+    @_last_op_log_host.setter
+    def _last_op_log_host(self, log):
+        self.__dict__["_last_op_log_host"] = log
 
     def _replay_flush(self, k_raw, v, positions, positions_host, counts, log, lengths, log_host, plans):
         """Re-apply one logged flush (litgpt/log_kv_cache.py:5067-5114) on the device.
@@ -805,7 +812,7 @@ class LogStructuredKVCache(nn.Module):
         """
         if lengths is None:
             raise ValueError("replay_op_log_len is required with replay_op_log")
-        if plans is not None and log_host is not plans.host_log:
+        if plans is not None and not plans.holds(log_host):
             raise RuntimeError("semantic replay plan does not match the CPU op-log")
         if self.semantic_unified_route:
             return self._unified_replay_flush(k_raw, v, positions, positions_host, counts, log, lengths, plans)
@@ -1316,8 +1323,9 @@ class LogKVStreamTrainingAttention(torch.autograd.Function):
                                      record_op_log=True, span_ends=None if ctx.span_ends is None else
                                      [row[start:end] for row in ctx.span_ends])
         op_log, op_log_len = cache.take_op_log()
-        ctx.replay_plans = _SemanticReplayPlans(cache._op_log_host)
-        ctx.op_log, ctx.op_log_len, ctx.op_log_host = op_log, op_log_len, ctx.replay_plans.host_log
+        # The log as taken: read through the property it would become lists.
+        ctx.op_log, ctx.op_log_len, ctx.op_log_host = op_log, op_log_len, cache.__dict__["_last_op_log_host"]
+        ctx.replay_plans = _SemanticReplayPlans(ctx.op_log_host)
         ctx.updates, ctx.plans, ctx.cache = updates, plans, cache
         ctx.scale, ctx.train_block, ctx.second_order_scale = scale, train_block, second_order_scale
         ctx.config = (cache.semantic_anchor_mode, cache.semantic_centroid_backend, cache.semantic_replay_updates,
