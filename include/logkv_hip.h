@@ -518,13 +518,14 @@ int logkv_decode_attention(const logkv_attention_args* args, const int32_t* tabl
  * current). No counterpart in the reference: it is for callers that cannot
  * allocate - code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc. Same arguments and result as logkv_decode_attention
- * (the same kernels); a call whose partials
- * (logkv_attention_workspace_bytes) exceed 16 MiB is rejected with
- * LOGKV_EINVAL. The stream must belong to the current device. Every call on
- * one GPU shares that GPU's scratch, so calls that overlap on one GPU (other
- * streams, other threads) race; serialize them. Each split writes its whole
- * partial before the combine reads it, so nothing needs clearing between
- * calls. */
+ * (the same kernels); a call is rejected with LOGKV_EINVAL when its partials
+ * (logkv_attention_workspace_bytes) exceed 16 MiB, and for more than 4 queries
+ * per KV group, dv above 128 or dk below 8 when n_batch * n_groups * queries per
+ * KV group * (dv + 2) floats for every 512 rows of cap do. The stream must
+ * belong to the current device. Every call on one GPU shares that GPU's
+ * scratch, so calls that overlap on one GPU (other streams, other threads)
+ * race; serialize them. Each split writes its whole partial before the combine
+ * reads it, so nothing needs clearing between calls. */
 int logkv_decode_attention_static(const logkv_attention_args* args, const int32_t* table, int64_t table_ints,
                                   void* stream);
 

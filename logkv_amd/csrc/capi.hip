@@ -237,7 +237,7 @@ int check_decode(const logkv_attention_args* a, const int32_t* table, int64_t ta
   if (a->n_batch < 1 || a->cap < 1 || a->tail < 0 || a->tail > a->cap)
     return fail(LOGKV_EINVAL, "attention needs n_batch >= 1 and 0 <= tail <= cap (cap >= 1)");
   if (!a->q || !a->k || !a->v || !a->out) return fail(LOGKV_EINVAL, "attention buffer is NULL");
-  // The streaming and tiled kernels read packed rows in 16-byte units.
+  // Packed rows are read in 16-byte units.
   if (reinterpret_cast<uintptr_t>(a->k) % 16 || reinterpret_cast<uintptr_t>(a->v) % 16)
     return fail(LOGKV_EINVAL, "packed K/V must be 16-byte aligned");
   return LOGKV_OK;
@@ -248,6 +248,18 @@ int check_decode(const logkv_attention_args* a, const int32_t* table, int64_t ta
 // life of the process; in host code the array's name is not a device address, so its
 // address is taken once per device with hipGetSymbolAddress and only that is used.
 constexpr int64_t kStaticScratchBytes = int64_t(16) << 20;
+
+// What a call of logkv_decode_attention_static is measured by: its partials, or for more than 4
+// queries per KV group, values wider than 128 or keys narrower than 8 one partial per 512 rows of
+// capacity where that is more. The launch needs less there; the bound is a contract of its own, so
+// that a capacity keeps being refused or accepted whatever the kernels split it into.
+int64_t static_decode_bytes(const logkv_attention_args& a) {
+  const int64_t nq = (a.n_heads / a.n_groups) * a.tq;
+  const bool few = nq <= 4 && a.dv <= 128 && a.dk >= 8;
+  const int64_t per_512 = few ? 0 : int64_t(a.n_batch) * a.n_groups * ((int64_t(a.cap) + 511) / 512) * nq * (a.dv + 2);
+  return std::max(logkv::attention_workspace_floats(a), per_512) * 4;
+}
+
 constexpr int kMaxScratchDevices = 64;
 }  // namespace
 
@@ -643,9 +655,9 @@ int logkv_decode_attention_static(const logkv_attention_args* a, const int32_t* 
                                   void* stream) {
   int rc = check_decode(a, table, table_ints);
   if (rc) return rc;
-  const int64_t need = logkv::attention_workspace_floats(*a) * 4;
+  const int64_t need = static_decode_bytes(*a);
   if (need > kStaticScratchBytes)
-    return fail(LOGKV_EINVAL, "decode partials need %lld bytes, above the static scratch of %lld bytes",
+    return fail(LOGKV_EINVAL, "decode partials are sized at %lld bytes, above the static scratch of %lld bytes",
                 (long long)need, (long long)kStaticScratchBytes);
   void* scratch_ptr = nullptr;
   rc = static_scratch(&scratch_ptr);

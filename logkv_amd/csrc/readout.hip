@@ -523,14 +523,9 @@ int attention_splits(const logkv_attention_args& a) {
   return std::max(1, std::min((a.cap + 127) / 128, blocks / std::max(1, lanes)));
 }
 
-// Partials of the launch, or for more than 4 queries or dv > 128 room for one per 512 rows of
-// capacity when that is more: the size (and with it what fits the static scratch) that callers
-// of those shapes were always asked for.
 int64_t attention_workspace_floats(const logkv_attention_args& a) {
   const int nq = (a.n_heads / a.n_groups) * a.tq;
-  const bool few = nq <= 4 && a.dv <= 128 && a.dk >= 8;
-  const int n_split = std::max(attention_splits(a), few ? 1 : (a.cap + 511) / 512);
-  return static_cast<int64_t>(a.n_batch) * a.n_groups * n_split * nq * (a.dv + 2);
+  return static_cast<int64_t>(a.n_batch) * a.n_groups * attention_splits(a) * nq * (a.dv + 2);
 }
 
 int launch_combine(const logkv_attention_args& a, const float* part, int n_split, hipStream_t stream) {

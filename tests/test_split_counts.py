@@ -1,4 +1,4 @@
-"""Key-range splits of the matrix-core attention, read off the workspace sizes the library asks for (no
+"""Key-range splits of the attention kernels, read off the workspace sizes the library asks for (no
 GPU needed): the count a launch takes is one of those that were fastest on an MI355X, also where a flat
 charge per split would trade a few tiles of the walk for gigabytes of float32 partials. Times beside each
 case are of the whole call, in us, by count."""
@@ -69,3 +69,17 @@ def test_forward_takes_a_fast_count(shape, fast):
 ])
 def test_backward_takes_a_fast_count(shape, fast):
     assert backward_parts(*shape) in fast
+
+
+@pytest.mark.parametrize("batch,groups,heads,tq,dk,dv,cap,splits", [
+    (8, 8, 64, 2, 128, 128, 16896, 8),      # 512 blocks over 64 lanes
+    (1, 2, 16, 2, 128, 128, 1000, 8),       # one per 128 rows
+    (1, 1, 4, 4, 256, 256, 40000, 256),     # values wider than 128: one block per CU
+    (1, 1, 4, 1, 4, 128, 40000, 313),
+    (600, 1, 1, 1, 64, 64, 5000, 1),
+])
+def test_decode_workspace_is_what_its_splits_fill(batch, groups, heads, tq, dk, dv, cap, splits):
+    a = _args(batch, groups, heads, tq, dv, cap)
+    a.dk, a.dim = dk, packed_dim(dk, dv)
+    need = _lib.lib().logkv_attention_workspace_bytes(C.byref(a))
+    assert need == batch * groups * splits * (heads // groups * tq) * (dv + 2) * 4

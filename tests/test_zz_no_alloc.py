@@ -1,8 +1,8 @@
 """The allocation-free decode entry point (logkv_decode_attention_static) against the
 workspace one (logkv_decode_attention), both called through the C ABI: the same
 kernels, so the outputs must be bit-identical, on two calls in a row - the second
-smaller, with another kernel path - and a call beyond the static scratch is refused
-before anything is launched."""
+smaller, with more queries per KV group - and a call beyond the static scratch's bound
+is refused before anything is launched."""
 
 from __future__ import annotations
 
@@ -71,13 +71,13 @@ def _both(cache, plan, q, ka, va, tail):
 
 
 def test_static_decode_equals_workspace_decode_twice():
-    # First call: batch 8 x 8 KV groups, 16 query heads, one query row (streaming kernel).
+    # First call: batch 8 x 8 KV groups, 16 query heads, one query row.
     big = _packed_case(8, 8, 16, 1, seed=3, max_seq=8192)
     out_ws, out_st = _both(*big)
     assert not torch.isnan(out_ws.float()).any()
     assert torch.equal(out_ws, out_st)
     # Second call, smaller: batch 2 x 4 KV groups, 16 heads, two query rows (8 queries per KV
-    # group: the tiled kernel). The scratch keeps the first call's partials; they must not leak.
+    # group). The scratch keeps the first call's partials; they must not leak.
     small = _packed_case(2, 4, 16, 2, seed=5, max_seq=4096)
     out_ws, out_st = _both(*small)
     assert not torch.isnan(out_ws.float()).any()
@@ -87,7 +87,8 @@ def test_static_decode_equals_workspace_decode_twice():
 def test_static_decode_refuses_more_than_its_scratch():
     lib = _lib.lib()
     dev = torch.device("cuda")
-    # 64 lanes x 16 queries per KV group over 16896 rows: 33 splits of partials, 17.6 MB > 16 MiB.
+    # 64 lanes x 16 queries per KV group over 16896 rows: one partial per 512 rows is 17.6 MB > 16 MiB, the
+    # bound of such calls (the launch itself writes 8 a lane).
     bt, G, heads, tq, cap, dim = 8, 8, 64, 2, 16896, 136
     ka = torch.zeros(bt, G, cap, dim, dtype=torch.bfloat16, device=dev)
     va = torch.zeros_like(ka)
@@ -95,9 +96,35 @@ def test_static_decode_refuses_more_than_its_scratch():
     out = torch.full((bt, heads, tq, 128), 7.0, dtype=torch.bfloat16, device=dev)
     table = torch.tensor([cap - 16], dtype=torch.int32, device=dev)
     a = _args(q, ka, va, cap - 16, 16, 128 ** -0.5, G, out)
-    assert lib.logkv_attention_workspace_bytes(C.byref(a)) > STATIC_SCRATCH_BYTES
+    assert 33 * bt * G * 16 * 130 * 4 > STATIC_SCRATCH_BYTES
+    assert lib.logkv_attention_workspace_bytes(C.byref(a)) == 8 * bt * G * 16 * 130 * 4
     rc = lib.logkv_decode_attention_static(C.byref(a), table.data_ptr(), 1, torch.cuda.current_stream().cuda_stream)
     assert rc == _lib.LOGKV_EINVAL
     assert "static scratch" in lib.logkv_last_error().decode()
     torch.cuda.synchronize()
     assert bool((out == 7.0).all())
+
+
+@pytest.mark.parametrize("cap,refused", [(31 * 512, False), (31 * 512 + 1, True)])
+def test_static_decode_bound(cap, refused):
+    """The last capacity that the bound accepts, with the workspace entry point's result, and the first it does not."""
+    print(f"case cap={cap}", flush=True)
+    lib, dev = _lib.lib(), torch.device("cuda")
+    bt, G, heads, tq, dim = 8, 8, 64, 2, 136
+    g = torch.Generator(device=dev).manual_seed(cap)
+    ka, va = (torch.randn(bt, G, cap, dim, generator=g, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(bt, heads, tq, 128, generator=g, device=dev, dtype=torch.bfloat16)
+    outs = [torch.full((bt, heads, tq, 128), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    table = torch.tensor([cap - 16], dtype=torch.int32, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    a_st, a_ws = (_args(q, ka, va, cap - 16, 16, 128 ** -0.5, G, out) for out in outs)
+    rc = lib.logkv_decode_attention_static(C.byref(a_st), table.data_ptr(), 1, stream)
+    need = lib.logkv_attention_workspace_bytes(C.byref(a_ws))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    _lib.check(lib.logkv_decode_attention(C.byref(a_ws), table.data_ptr(), 1, ws.data_ptr(), need, stream), "decode")
+    torch.cuda.synchronize()
+    if refused:
+        assert rc == _lib.LOGKV_EINVAL and bool((outs[0] == 7.0).all())
+    else:
+        assert rc == 0 and torch.equal(*outs)
+    assert bool(torch.isfinite(outs[1].float()).all())
