@@ -451,19 +451,22 @@ __global__ __launch_bounds__(256) void slot_pack_kernel(logkv_slot_pack_args a) 
 
 // The rows a decode step adds to a packed prefix: recent rows from recent_start on and the
 // current rows, copied with a zero bias (they are valid and carry their own rotation). One
-// thread per 4-feature unit; the only dependent load is the prefix length. A general pack block
-// resolves 64 row sources through the plan first: one row of 8 lanes 5.7 -> 2.9 us, of 64 lanes
-// 9.0 -> 3.9 us.
+// thread per F-feature unit (8 where every row allows 16-byte accesses, else 4); the only
+// dependent load is the prefix length. A general pack block resolves 64 row sources through the
+// plan first: one row of 8 lanes 5.7 -> 2.9 us, of 64 lanes 9.0 -> 3.9 us; 501 rows of 512 lanes
+// 69 us, in 4-feature units 76 us, in 8-feature ones 51 us.
+template <int F>
 __global__ __launch_bounds__(256) void pack_tail_kernel(logkv_readout_view c, logkv_pack_args p,
                                                         const int32_t* __restrict__ width_ptr) {
+  using Unit = std::conditional_t<F == 8, uint4, uint2>;
   const int lane = blockIdx.y, b = lane / c.n_groups, g = lane % c.n_groups;
-  const int units = p.dim / 4, new_recent = c.recent_count - p.recent_start, rows = new_recent + p.cur_len;
+  const int units = p.dim / F, new_recent = c.recent_count - p.recent_start, rows = new_recent + p.cur_len;
   const int first = *width_ptr + (c.alpha_count_dev ? *c.alpha_count_dev : c.alpha_count) + p.recent_start;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= rows * 2 * units) return;
   const int r = i / (2 * units), e = i - r * 2 * units;
   const bool key = e < units;
-  const int d = 4 * (key ? e : e - units), n = key ? c.dk : c.dv;
+  const int d = F * (key ? e : e - units), n = key ? c.dk : c.dv;
   const LOGKV_G uint16_t* src;
   if (r < new_recent) {
     const int64_t row = static_cast<int64_t>(lane) * c.recent_cap + p.recent_start + r;
@@ -472,11 +475,20 @@ __global__ __launch_bounds__(256) void pack_tail_kernel(logkv_readout_view c, lo
     const int64_t t = r - new_recent;
     src = key ? gp(p.cur_k) + b * p.ck_sb + g * p.ck_sg + t * p.ck_st : gp(p.cur_v) + b * p.cv_sb + g * p.cv_sg + t * p.cv_st;
   }
-  uint2 x = make_uint2(0u, 0u);
-  if (d < n) x = *reinterpret_cast<const LOGKV_G uint2*>(src + d);
+  Unit x{};
+  if (d < n) x = *reinterpret_cast<const LOGKV_G Unit*>(src + d);
   if (first + r >= p.out_cap) return;
-  *reinterpret_cast<LOGKV_G uint2*>((key ? gp(p.out_k) : gp(p.out_v)) +
-                                    (static_cast<int64_t>(lane) * p.out_cap + first + r) * p.dim + d) = x;
+  *reinterpret_cast<LOGKV_G Unit*>((key ? gp(p.out_k) : gp(p.out_v)) +
+                                   (static_cast<int64_t>(lane) * p.out_cap + first + r) * p.dim + d) = x;
+}
+
+// Whether every row that the tail pack reads and writes starts at a multiple of F features (2 F bytes).
+template <int F>
+bool tail_units(const logkv_readout_view& c, const logkv_pack_args& p) {
+  auto at = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % (2 * F) == 0; };
+  const bool cur = !p.cur_len || (at(p.cur_k) && at(p.cur_v) && p.ck_sb % F == 0 && p.ck_sg % F == 0 && p.ck_st % F == 0 &&
+                                  p.cv_sb % F == 0 && p.cv_sg % F == 0 && p.cv_st % F == 0);
+  return c.dk % F == 0 && c.dv % F == 0 && at(c.recent_k) && at(c.recent_v) && at(p.out_k) && at(p.out_v) && cur;
 }
 
 }  // namespace
@@ -501,12 +513,11 @@ int launch_pack(const logkv_readout_view& c, const logkv_pack_args& p, const int
   const int rows = p.skip_pooled ? c.recent_count + p.cur_len - p.recent_start : p.out_cap;
   if (rows <= 0) return LOGKV_OK;
   const int lanes = c.n_batch * c.n_groups;
-  const bool units4 = c.dk % 4 == 0 && c.dv % 4 == 0 && reinterpret_cast<uintptr_t>(c.recent_k) % 8 == 0 &&
-                      reinterpret_cast<uintptr_t>(c.recent_v) % 8 == 0;
-  if (p.skip_pooled && !p.out_w && units4) {
-    const int items = rows * 2 * (p.dim / 4);
-    hipLaunchKernelGGL(pack_tail_kernel, dim3((items + 255) / 256, lanes), dim3(256), 0, stream, c, p,
-                       table + static_cast<int64_t>(lanes) * (c.k_max * c.levels + 1));
+  if (p.skip_pooled && !p.out_w && tail_units<4>(c, p)) {
+    const bool wide = tail_units<8>(c, p);
+    const int items = rows * 2 * (p.dim / (wide ? 8 : 4));
+    hipLaunchKernelGGL(wide ? pack_tail_kernel<8> : pack_tail_kernel<4>, dim3((items + 255) / 256, lanes), dim3(256), 0,
+                       stream, c, p, table + static_cast<int64_t>(lanes) * (c.k_max * c.levels + 1));
     return hipGetLastError() == hipSuccess ? LOGKV_OK : LOGKV_ERUNTIME;
   }
   // Tiles past the packed rows (known on the device only) exit at once.
