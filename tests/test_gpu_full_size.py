@@ -1,7 +1,7 @@
 """Parity at the benchmarked sizes, where the kernels take the geometry they run in the benchmark:
 
 * decode at batch 8 over a 32K-token Qwen3-1.7B cache (64 lanes of about 8.8K packed rows, so the
-  streaming kernel splits each lane 20 ways), every output against the oracle's float64 attention;
+  kernel splits each lane 8 ways and a block walks nine 128-row passes), every output against the oracle's float64 attention;
 * chunk attention of one 2048-token prefill block, 16 query heads, over a state of more than 5K
   packed rows per lane (key ranges split over many blocks), sampled query rows of three KV groups
   against the oracle;

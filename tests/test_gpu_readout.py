@@ -186,15 +186,15 @@ def test_decode_qwen_shape():
 
 @pytest.mark.parametrize("dk,dv,heads,groups,tq", [
     (128, 128, 8, 8, 1),    # one query per KV group; the bias column starts a 16-byte unit of its own
-    (120, 120, 6, 2, 1),    # three queries per group (one idle query slot)
+    (120, 120, 6, 2, 1),    # three queries per group
     (128, 128, 8, 2, 1),    # four queries per group
     (60, 60, 4, 2, 1),      # dk not a multiple of 8: the bias shares a unit with the last key features
-    (200, 104, 2, 2, 1),    # two key units per lane, narrower values
-    (132, 128, 2, 2, 2),    # two current rows (causal), bias sharing a unit, two key units per lane
+    (200, 104, 2, 2, 1),    # packed width above 160, values of a partial 16-wide block
+    (132, 128, 2, 2, 2),    # two current rows (causal), bias sharing a unit
 ])
 def test_streaming_decode_shapes(dk, dv, heads, groups, tq):
-    """Decode steps of up to 4 query rows per KV group take the streaming kernel; every variant of it
-    (queries per group, key units per lane, bias column on its own or not) against the oracle."""
+    """Decode steps of up to 4 query rows per KV group: query counts, packed widths and the bias column
+    in a 16-byte unit of its own or not, against the oracle."""
     print(f"case dk={dk} dv={dv} heads={heads} groups={groups} tq={tq}", flush=True)
     cos, sin = rope_tables(2048, dk)
     cache = LogStructuredKVCache(
